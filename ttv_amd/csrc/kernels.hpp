@@ -15,7 +15,8 @@
 //           item; partial sums over k meet by recursive halving (one wave) or in LDS (several
 //           waves).  Outputs leave with non-temporal stores where one wave instruction writes
 //           whole 128-byte lines (BF16/FP8 lane vectors are first transposed through LDS).
-//   k_strided  general strides that do not fold to three dimensions: one thread per output.
+//   k_strided  general strides that do not fold to three dimensions and have no unit-stride dimension
+//           (view.hpp has the ones that do): one thread per output.
 //   k_finalize sums the split-n_q partials (FP32 or FP64) and applies FP8 scales.
 //
 // Storage types: float, double, bfloat16 (uint16_t) and OCP FP8-e4m3 (uint8_t).  Accumulation
@@ -446,23 +447,22 @@ __device__ __forceinline__ bool halving_sum_ct(Acc (&v)[N], int lane, int& base,
 	return (lane & (kRest - 1)) == 0;
 }
 
-// FP8 scales of the VEC consecutive outputs (o, i .. i+VEC-1), one group-index division per vector
+// FP8 scales of the VEC consecutive outputs numbered j0 .. j0+VEC-1, one group-index division per vector
 template<typename Acc, int VEC>
-__device__ __forceinline__ void scale_vec(const Args& P, int64_t o, int64_t i, Acc (&w)[VEC])
+__device__ __forceinline__ void scale_vec(const float* __restrict__ scales, int64_t fps, int64_t j0, Acc (&w)[VEC])
 {
-	if(P.scales == nullptr) return;
-	int64_t const j0 = o * P.I + i;
-	int64_t const g0 = j0 / P.fps;
-	if(P.fps >= VEC) {
+	if(scales == nullptr) return;
+	int64_t const g0 = j0 / fps;
+	if(fps >= VEC) {
 		// at most one group boundary inside the vector
-		int64_t const rem = j0 - g0 * P.fps;
-		Acc const s0 = static_cast<Acc>(P.scales[g0]);
-		Acc const s1 = rem + VEC > P.fps ? static_cast<Acc>(P.scales[g0 + 1]) : s0;
+		int64_t const rem = j0 - g0 * fps;
+		Acc const s0 = static_cast<Acc>(scales[g0]);
+		Acc const s1 = rem + VEC > fps ? static_cast<Acc>(scales[g0 + 1]) : s0;
 #pragma unroll
-		for(int e = 0; e < VEC; ++e) w[e] *= rem + e < P.fps ? s0 : s1;
+		for(int e = 0; e < VEC; ++e) w[e] *= rem + e < fps ? s0 : s1;
 	} else {
 #pragma unroll
-		for(int e = 0; e < VEC; ++e) w[e] *= static_cast<Acc>(P.scales[(j0 + e) / P.fps]);
+		for(int e = 0; e < VEC; ++e) w[e] *= static_cast<Acc>(scales[(j0 + e) / fps]);
 	}
 }
 
@@ -488,7 +488,7 @@ __device__ __forceinline__ void store_vec(void* __restrict__ C, const Args& P, i
 	Acc w[VEC];
 #pragma unroll
 	for(int e = 0; e < VEC; ++e) w[e] = v[e];
-	if constexpr(SC) scale_vec<Acc, VEC>(P, o, i, w);
+	if constexpr(SC) scale_vec<Acc, VEC>(P.scales, P.fps, o * P.I + i, w);
 	Acc* dst = static_cast<Acc*>(C) + o * P.sCo + i;
 	if(P.cvec == 0 || (BYTES >= 16 ? P.cvec < 16 : P.cvec < BYTES)) {
 		// C rows off the vector grid (a row length that 4 outputs do not divide): element-aligned
@@ -611,7 +611,7 @@ __device__ __forceinline__ void col_store_transposed(void* __restrict__ C, const
 #pragma unroll
 		for(int e = 0; e < VEC; ++e) w[e] = v[u][e];
 		if constexpr(SC)
-			if(row_ok && ii < P.I) scale_vec<Acc, VEC>(P, oo, ii, w);
+			if(row_ok && ii < P.I) scale_vec<Acc, VEC>(P.scales, P.fps, oo * P.I + ii, w);
 		// the previous unit's reads of the slice are done before it is written again
 		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 		__builtin_amdgcn_wave_barrier();
@@ -1389,6 +1389,12 @@ struct StridedArgs {
 	int64_t K, sAk, outputs;
 	const float* scales;
 	int64_t fps;
+	// k_view_cols: vector units of all outer indices, contraction groups per block; k_view_rows: lanes per row
+	int64_t units;
+	int     ks, lpr;
+	// division by the extents (by the vectors of a row in place of n[0] for k_view_cols) when indices fit 31 bits
+	int     idx32;
+	uint32_t mul[kMaxFree], sh[kMaxFree];
 };
 
 template<typename S, bool KAHAN>

@@ -6,6 +6,7 @@
 #include <algorithm>
 
 #include "runtime.hpp"
+#include "view.hpp"
 
 namespace ttvx
 {
@@ -101,11 +102,32 @@ int launch_width(const Config& cfg, const S* A, const typename Traits<S>::acc* B
 	else return fail(TTVX_ERR_UNSUPPORTED, "ttvx: unsupported vector width");
 }
 
+// Views that do not fold (view.hpp)
+template<typename S, bool KH, int V>
+int launch_view(const Config& cfg, const S* A, const typename Traits<S>::acc* B, void* C, hipStream_t s)
+{
+	if constexpr(V > 1)
+		if(cfg.vec != V) return launch_view<S, KH, V / 2>(cfg, A, B, C, s);
+	dim3 const grid(static_cast<unsigned>(cfg.grid)), block(kBlock);
+	if(cfg.lean == LEAN_VIEW_COLS)
+		hipLaunchKernelGGL((k_view_cols<S, V, KH>), grid, block, cfg.shmem, s, A, B, C, cfg.sargs);
+	else if(cfg.lean == LEAN_VIEW_LONG_ROWS)
+		hipLaunchKernelGGL((k_view_long_rows<S, V, KH>), grid, block, 0, s, A, B, C, cfg.sargs);
+	else if(cfg.U == 8)
+		hipLaunchKernelGGL((k_view_rows<S, V, 8, KH>), grid, block, 0, s, A, B, C, cfg.sargs);
+	else if(cfg.U == 2)
+		hipLaunchKernelGGL((k_view_rows<S, V, 2, KH>), grid, block, 0, s, A, B, C, cfg.sargs);
+	else
+		hipLaunchKernelGGL((k_view_rows<S, V, 1, KH>), grid, block, 0, s, A, B, C, cfg.sargs);
+	return TTVX_OK;
+}
+
 template<typename S, bool KH>
 int launch_kh(const Config& cfg, const S* A, const typename Traits<S>::acc* B, void* C, hipStream_t s)
 {
 	if(cfg.kind == KIND_STRIDED) {
 		if constexpr(!kRealigned<S>) {
+			if(cfg.lean != LEAN_NONE) return launch_view<S, KH, Traits<S>::vmax>(cfg, A, B, C, s);
 			hipLaunchKernelGGL((k_strided<S, KH>), dim3(static_cast<unsigned>(cfg.grid)), dim3(kBlock), 0, s, A, B, C, cfg.sargs);
 			return TTVX_OK;
 		}

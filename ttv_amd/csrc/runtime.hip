@@ -230,6 +230,65 @@ constexpr int kDotGridPerCU = 64;
 constexpr int64_t kNarrowLanes = TTVX_NARROW_LANES;
 } // namespace
 
+namespace
+{
+// The strided variant's unit-stride kernels (view.hpp) where they apply: columns when the fastest free
+// dimension has unit stride in A and C, else rows when the contraction has.
+void configure_view(const Fold& f, const DType& dt, Config& cfg)
+{
+	StridedArgs& G = cfg.sargs;
+	int64_t const waves_wanted = static_cast<int64_t>(cfg.cus) * 8;
+	G.idx32 = G.outputs < (int64_t{1} << 31) ? 1 : 0;
+	auto fast_div = [&G](int d, int64_t n) {
+		if(!G.idx32) return;
+		uint32_t l = 0;
+		while((int64_t{1} << l) < n) ++l;
+		G.mul[d] = static_cast<uint32_t>((((uint64_t{1} << l) - static_cast<uint64_t>(n)) << 32) / static_cast<uint64_t>(n) + 1);
+		G.sh[d] = l;
+	};
+	for(int d = 0; d < G.nd; ++d) fast_div(d, G.n[d]);
+	if(G.nd >= 1 && G.sa[0] == 1 && G.sc[0] == 1 && G.n[0] > 1) {
+		int const vec = pick_vec(dt, G.n[0]);
+		int64_t const units = G.outputs / G.n[0] * ceil_div(G.n[0], vec);
+		// contraction groups only while the units alone leave the chip short of waves: 8 waves per CU with
+		// 8 loads each cover the memory latency; a group keeps at least one round of loads
+		int ks = 1;
+		while(ks < 16 && units * ks < waves_wanted * 64 && f.K / (2 * ks) >= 8) ks *= 2;
+		int64_t const blocks = ceil_div(units, kBlock / ks);
+		if(blocks > kMaxLeanBlocks) return;
+		fast_div(0, ceil_div(G.n[0], vec));
+		G.units = units;
+		G.ks = ks;
+		cfg.vec = vec;
+		cfg.lean = LEAN_VIEW_COLS;
+		cfg.grid = static_cast<int>(blocks);
+		cfg.shmem = ks > 1 ? static_cast<std::size_t>(kBlock) * vec * acc_size(dt) : 0;
+	} else if(f.sAk == 1 && f.K > 1) {
+		int const vec = pick_vec(dt, f.K);
+		int64_t const vsteps = ceil_div(f.K, vec);
+		int64_t blocks;
+		if(vsteps <= 64) {
+			G.lpr = static_cast<int>(vsteps);
+			int64_t const rpw = 64 / vsteps;
+			// row sets per wave: as many loads in flight as leave 8 waves per CU
+			cfg.U = f.outputs >= waves_wanted * rpw * 8 ? 8 : (f.outputs >= waves_wanted * rpw * 2 ? 2 : 1);
+			blocks = ceil_div(f.outputs, rpw * cfg.U * (kBlock / 64));
+			cfg.lean = LEAN_VIEW_ROWS;
+		} else {
+			G.lpr = f.outputs < waves_wanted && vsteps >= 2 * kBlock ? kBlock : 64;
+			blocks = ceil_div(f.outputs, kBlock / G.lpr);
+			cfg.lean = LEAN_VIEW_LONG_ROWS;
+		}
+		if(blocks > kMaxLeanBlocks) {
+			cfg.lean = LEAN_NONE;
+			return;
+		}
+		cfg.vec = vec;
+		cfg.grid = static_cast<int>(blocks);
+	}
+}
+} // namespace
+
 bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus, unsigned flags, Config& cfg)
 {
 	cfg = Config{};
@@ -250,6 +309,7 @@ bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus,
 		for(int d = 0; d < G.nd; ++d) { G.n[d] = f.dims[d].n; G.sa[d] = f.dims[d].sa; G.sc[d] = f.dims[d].sc; }
 		G.K = f.K; G.sAk = f.sAk; G.outputs = f.outputs; G.fps = 1;
 		cfg.grid = static_cast<int>(std::max<int64_t>(1, std::min(ceil_div(f.outputs, kBlock), gridcap)));
+		configure_view(f, dt, cfg);
 		return true;
 	}
 	if(!f.three_d) return false;

@@ -28,6 +28,8 @@
 
 #include <type_traits>
 
+#include "fastdiv.hpp"
+
 namespace ttvx
 {
 
@@ -1394,7 +1396,7 @@ struct StridedArgs {
 	int     ks, lpr;
 	// division by the extents (by the vectors of a row in place of n[0] for k_view_cols) when indices fit 31 bits
 	int     idx32;
-	uint32_t mul[kMaxFree], sh[kMaxFree];
+	FastDiv div[kMaxFree];
 };
 
 template<typename S, bool KAHAN>

@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "fastdiv.hpp"
+
 namespace ttvx
 {
 
@@ -50,6 +52,12 @@ struct QuantArgs {
 	int64_t sAo, sAk, sAi;
 	int64_t fps;          // fibers per scale group
 	int64_t groups;
+	// k_quant_tile / k_quant_cols: fibers and groups per block, lanes along fiber vectors and along k, fiber vectors
+	// per thread, k steps per lane; k_quant_cols / k_quant_long: contraction rows / values per block
+	int64_t nf;
+	int tile_groups, LV, KS, F, steps;
+	int64_t kchunk;
+	FastDiv by_slab, by_I, by_fps;      // k_quant_slabs: division by K*I, I and fps
 };
 
 } // namespace ttvx

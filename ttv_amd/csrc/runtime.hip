@@ -239,14 +239,8 @@ void configure_view(const Fold& f, const DType& dt, Config& cfg)
 	StridedArgs& G = cfg.sargs;
 	int64_t const waves_wanted = static_cast<int64_t>(cfg.cus) * 8;
 	G.idx32 = G.outputs < (int64_t{1} << 31) ? 1 : 0;
-	auto fast_div = [&G](int d, int64_t n) {
-		if(!G.idx32) return;
-		uint32_t l = 0;
-		while((int64_t{1} << l) < n) ++l;
-		G.mul[d] = static_cast<uint32_t>((((uint64_t{1} << l) - static_cast<uint64_t>(n)) << 32) / static_cast<uint64_t>(n) + 1);
-		G.sh[d] = l;
-	};
-	for(int d = 0; d < G.nd; ++d) fast_div(d, G.n[d]);
+	if(G.idx32)
+		for(int d = 0; d < G.nd; ++d) G.div[d] = fast_div(G.n[d]);
 	if(G.nd >= 1 && G.sa[0] == 1 && G.sc[0] == 1 && G.n[0] > 1) {
 		int const vec = pick_vec(dt, G.n[0]);
 		int64_t const units = G.outputs / G.n[0] * ceil_div(G.n[0], vec);
@@ -256,7 +250,7 @@ void configure_view(const Fold& f, const DType& dt, Config& cfg)
 		while(ks < 16 && units * ks < waves_wanted * 64 && f.K / (2 * ks) >= 8) ks *= 2;
 		int64_t const blocks = ceil_div(units, kBlock / ks);
 		if(blocks > kMaxLeanBlocks) return;
-		fast_div(0, ceil_div(G.n[0], vec));
+		if(G.idx32) G.div[0] = fast_div(ceil_div(G.n[0], vec));
 		G.units = units;
 		G.ks = ks;
 		cfg.vec = vec;

@@ -21,12 +21,6 @@
 namespace ttvx
 {
 
-// x / d for x < 2^31 by the multiply and shift of Granlund and Montgomery (1994), mul and sh from fast_div
-__device__ __forceinline__ uint32_t div_by(uint32_t x, uint32_t mul, uint32_t sh)
-{
-	return (__umulhi(mul, x) + x) >> sh;
-}
-
 // A and C offsets of outer index o over the dimensions first .. nd-1 (fastest first)
 __device__ __forceinline__ void view_offsets(const StridedArgs& G, int first, int64_t o, int64_t& offa, int64_t& offc)
 {
@@ -35,7 +29,7 @@ __device__ __forceinline__ void view_offsets(const StridedArgs& G, int first, in
 	if(G.idx32) {
 		uint32_t rest = static_cast<uint32_t>(o);
 		for(int d = first; d < G.nd; ++d) {
-			uint32_t const q = div_by(rest, G.mul[d], G.sh[d]);
+			uint32_t const q = div_by(rest, G.div[d]);
 			uint32_t const idx = rest - q * static_cast<uint32_t>(G.n[d]);
 			rest = q;
 			offa += static_cast<int64_t>(idx) * G.sa[d];
@@ -72,7 +66,7 @@ __global__ __launch_bounds__(kBlock) void k_view_cols(const S* __restrict__ A, c
 	int64_t const unit = static_cast<int64_t>(blockIdx.x) * ul + l;
 	bool const live = unit < G.units;
 	int64_t const uc = live ? unit : G.units - 1;            // tail lanes re-read live data and store nothing
-	int64_t const o = G.idx32 ? static_cast<int64_t>(div_by(static_cast<uint32_t>(uc), G.mul[0], G.sh[0])) : uc / iv;
+	int64_t const o = G.idx32 ? static_cast<int64_t>(div_by(static_cast<uint32_t>(uc), G.div[0])) : uc / iv;
 	int64_t const i  = (uc - o * iv) * VEC;
 	int64_t const ic = i + VEC <= I ? i : I - VEC;           // a row's last vector is clamped to its end
 	int64_t offa, offc;

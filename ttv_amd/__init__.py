@@ -15,8 +15,14 @@ Everything runs in libttvx.so (HIP kernels for gfx950).  There is no CPU fallbac
 built library or without a GPU the calls raise.
 """
 import ctypes
+import functools
 
 import numpy as np
+
+try:
+    import torch
+except ImportError:                   # numpy alone is enough for the synchronous entry points
+    torch = None
 
 from . import _lib
 from ._lib import (BF16, F32, F64, FLAG_FP64_FINAL, FLAG_KAHAN, FP8E4M3, SELECT_AUTO, SELECT_FORCED,
@@ -34,11 +40,7 @@ __all__ = [
 
 
 def _is_torch(x):
-    try:
-        import torch
-        return isinstance(x, torch.Tensor)
-    except ImportError:
-        return False
+    return torch is not None and isinstance(x, torch.Tensor)
 
 
 def _describe(x):
@@ -52,8 +54,33 @@ def _describe(x):
 
 
 def _stream_ptr():
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream of the current device (the raw handle: building a Stream object takes 2.7 us)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+class _Plan:
+    """What a product's call needs besides its data: C's extents and strides and the library's argument arrays."""
+    __slots__ = ("nc", "wc", "na_", "wa_", "pia_", "nb_", "nc_", "wc_", "pic_", "K")
+
+    def __init__(self, q, na, wa):
+        pia = layout_from_strides(na, wa)
+        pic = generate_output_layout(pia, q)
+        self.nc = generate_output_shape(na, q)
+        self.wc = generate_strides(self.nc, pic)
+        self.K = int(na[q - 1])
+        self.na_, self.wa_, self.pia_, self.nb_ = sizes(na), sizes(wa), sizes(pia), sizes([self.K])
+        self.nc_, self.wc_, self.pic_ = sizes(self.nc), sizes(self.wc), sizes(pic)
+
+
+@functools.lru_cache(maxsize=1024)
+def _plan(q, na, wa):
+    """The plan of products over mode q of tensors with these extents and strides (a function of the three numbers
+    alone; the arrays are only read), or None when the arguments are not valid.  A call with a plan at hand takes
+    7 us of host time, one that builds it 15 us."""
+    p = len(na)
+    if p < 2 or not 1 <= q <= p or 0 in na:
+        return None
+    return _Plan(q, na, wa)
 
 
 def _vector(b, name="b"):
@@ -85,6 +112,21 @@ def ttv(q, A, b, *, flags=0, out=None):
     """C = A x_q b (q one-based).  C has A's shape without mode q and the reference's output
     layout (layout.h:143-207: A's layout with q removed) with dense strides.  b is a 1-D vector of
     A's element type (a strided b is copied); a given `out` must have C's shape and A's type."""
+    if _is_torch(A) and _is_torch(b) and A.is_cuda and b.is_cuda and out is None and isinstance(q, int):
+        dtype = A.dtype
+        if (dtype is torch.float32 or dtype is torch.float64) and b.dtype is dtype and b.dim() == 1:
+            plan = _plan(q, A.shape, A.stride())
+            if plan is not None and b.shape[0] == plan.K:
+                if b.stride(0) != 1:
+                    b = b.contiguous()
+                out = torch.empty_strided(plan.nc, plan.wc, dtype=dtype, device=A.device)
+                L = lib()
+                fn = L.ttvx_ttv_f32_async if dtype is torch.float32 else L.ttvx_ttv_f64_async
+                status = fn(q, len(plan.na_), A.data_ptr(), plan.na_, plan.wa_, plan.pia_, b.data_ptr(), plan.nb_,
+                            out.data_ptr(), plan.nc_, plan.wc_, plan.pic_, flags, _stream_ptr())
+                if status:
+                    check(status)
+                return out
     na, wa, pa, dt, dev = _describe(A)
     b = _vector(b)
     nb, _, pb, dtb, devb = _describe(b)
@@ -104,7 +146,6 @@ def ttv(q, A, b, *, flags=0, out=None):
     wc = generate_strides(nc, pic)
     if out is None:
         if _is_torch(A):
-            import torch
             out = torch.empty_strided(nc, wc, dtype=A.dtype, device=A.device)
         else:
             npdt = np.float32 if dt == "float32" else np.float64
@@ -196,7 +237,6 @@ def ttvs(q, A, bs, order="optimal"):
 def _kron(vectors, like):
     """Kronecker product of 1-D GPU vectors (vector 0 varies fastest), in like's dtype and device
     (a single vector is returned as it is)."""
-    import torch
     vs = [_vector(torch.as_tensor(v, device=like.device, dtype=like.dtype)) for v in vectors]
     if len(vs) == 1:
         return vs[0]
@@ -240,7 +280,6 @@ def _ttvs_fused(q, A, bs):
 
 def quantize_bf16(A):
     """bfloat16 bits (torch.uint16 tensor with A's shape and strides), round to nearest even."""
-    import torch
     if not (A.is_cuda and A.dtype == torch.float32):
         raise TTVError(_lib.ERR_ARGUMENT, "ttv_amd.quantize_bf16: A must be a float32 GPU tensor")
     na, wa = list(A.shape), list(A.stride())
@@ -259,70 +298,64 @@ def default_fibers_per_scale(K):
 
 def quantize_fp8(q, A, fibers_per_scale=None):
     """(codes, scales, fibers_per_scale): e4m3 codes with A's strides and per-group scales."""
-    import torch
     if not (A.is_cuda and A.dtype == torch.float32):
         raise TTVError(_lib.ERR_ARGUMENT, "ttv_amd.quantize_fp8: A must be a float32 GPU tensor")
-    na, wa = list(A.shape), list(A.stride())
-    pia = layout_from_strides(na, wa)
+    na, wa = A.shape, A.stride()
+    plan = _plan(q, na, wa)
+    na_, wa_, pia_ = (plan.na_, plan.wa_, plan.pia_) if plan is not None else \
+        (sizes(na), sizes(wa), sizes(layout_from_strides(na, wa)))
     fps = fibers_per_scale or default_fibers_per_scale(na[q - 1])
-    ns = lib().ttvx_fp8_num_scales(q, len(na), sizes(na), sizes(wa), sizes(pia), fps)
+    ns = lib().ttvx_fp8_num_scales(q, len(na), na_, wa_, pia_, fps)
     if ns == 0:
         check(_lib.ERR_ARGUMENT)
     span = 1 + sum((n - 1) * w for n, w in zip(na, wa))
     codes = torch.empty(span, dtype=torch.uint8, device=A.device)
     scales = torch.empty(ns, dtype=torch.float32, device=A.device)
-    check(lib().ttvx_quantize_fp8_async(q, len(na), ctypes.c_void_p(A.data_ptr()), sizes(na), sizes(wa), sizes(pia),
-                                        ctypes.c_void_p(codes.data_ptr()), ctypes.c_void_p(scales.data_ptr()), fps,
-                                        _stream_ptr()))
+    check(lib().ttvx_quantize_fp8_async(q, len(na), A.data_ptr(), na_, wa_, pia_, codes.data_ptr(), scales.data_ptr(),
+                                        fps, _stream_ptr()))
     return codes.as_strided(na, wa), scales, fps
 
 
 def _quantised_operands(q, Aq, storage, b, out, what):
-    """Checked (na, wa, pia, b, C, nc, wc, pic) of a reduced-precision product: Aq a GPU tensor of
+    """Checked (plan, b's extent, b, C, C's strides) of a reduced-precision product: Aq a GPU tensor of
     the storage type, b a float32 GPU vector (copied when strided), C float32 of C's shape."""
-    import torch
     if not (_is_torch(Aq) and Aq.is_cuda and Aq.dtype == storage):
         raise TTVError(_lib.ERR_ARGUMENT, "ttv_amd.%s: A must be a %s GPU tensor" % (what, str(storage).replace("torch.", "")))
-    na, wa = list(Aq.shape), list(Aq.stride())
+    na, wa = Aq.shape, Aq.stride()
     if not (1 <= q <= len(na)):
         raise TTVError(_lib.ERR_ARGUMENT, "Error in tlib::tensor_times_vector: contraction mode should be greater zero or less than or equal to p.")
-    pia = layout_from_strides(na, wa)
     if not _is_torch(b) or not b.is_cuda or b.dtype != torch.float32:
         raise TTVError(_lib.ERR_ARGUMENT, "ttv_amd.%s: b must be a float32 GPU vector" % what)
     b = _vector(b)
-    nc = generate_output_shape(na, q)
-    pic = generate_output_layout(pia, q)
+    plan = _plan(q, na, wa) or _Plan(q, na, wa)      # the library reports what is not valid
+    nb_ = plan.nb_ if b.shape[0] == plan.K else sizes([b.shape[0]])
+    wc_ = plan.wc_
     if out is None:
-        wc = generate_strides(nc, pic)
-        out = torch.empty_strided(nc, wc, dtype=torch.float32, device=Aq.device)
+        out = torch.empty_strided(plan.nc, plan.wc, dtype=torch.float32, device=Aq.device)
     else:
         if not _is_torch(out):
             raise TTVError(_lib.ERR_ARGUMENT, "ttv_amd.%s: out must be a GPU tensor" % what)
-        wc = _checked_out(out, nc, "float32", True)
-    return na, wa, pia, b, out, nc, wc, pic
+        wc_ = sizes(_checked_out(out, plan.nc, "float32", True))
+    return plan, nb_, b, out, wc_
 
 
 def ttv_bf16(q, Aq, b, *, flags=0, out=None):
     """C = A x_q b for bfloat16 A (torch.uint16 bits), float32 b and C."""
-    import torch
-    na, wa, pia, b, c, nc, wc, pic = _quantised_operands(q, Aq, torch.uint16, b, out, "ttv_bf16")
-    check(lib().ttvx_ttv_bf16_async(q, len(na), ctypes.c_void_p(Aq.data_ptr()), sizes(na), sizes(wa), sizes(pia),
-                                    ctypes.c_void_p(b.data_ptr()), sizes([b.shape[0]]), ctypes.c_void_p(c.data_ptr()),
-                                    sizes(nc), sizes(wc), sizes(pic), flags, _stream_ptr()))
+    plan, nb_, b, c, wc_ = _quantised_operands(q, Aq, torch.uint16, b, out, "ttv_bf16")
+    check(lib().ttvx_ttv_bf16_async(q, len(Aq.shape), Aq.data_ptr(), plan.na_, plan.wa_, plan.pia_, b.data_ptr(), nb_,
+                                    c.data_ptr(), plan.nc_, wc_, plan.pic_, flags, _stream_ptr()))
     return c
 
 
 def ttv_fp8(q, codes, scales, fibers_per_scale, b, *, flags=0, out=None):
     """C = A x_q b for e4m3 A (codes + scales from quantize_fp8), float32 b and C."""
-    import torch
-    na, wa, pia, b, c, nc, wc, pic = _quantised_operands(q, codes, torch.uint8, b, out, "ttv_fp8")
+    plan, nb_, b, c, wc_ = _quantised_operands(q, codes, torch.uint8, b, out, "ttv_fp8")
     if not (_is_torch(scales) and scales.is_cuda and scales.dtype == torch.float32 and scales.dim() == 1):
         raise TTVError(_lib.ERR_ARGUMENT, "ttv_amd.ttv_fp8: scales must be a float32 GPU vector")
     scales = _vector(scales, "scales")
-    check(lib().ttvx_ttv_fp8_async(q, len(na), ctypes.c_void_p(codes.data_ptr()), sizes(na), sizes(wa), sizes(pia),
-                                   ctypes.c_void_p(scales.data_ptr()), fibers_per_scale,
-                                   ctypes.c_void_p(b.data_ptr()), sizes([b.shape[0]]), ctypes.c_void_p(c.data_ptr()),
-                                   sizes(nc), sizes(wc), sizes(pic), flags, _stream_ptr()))
+    check(lib().ttvx_ttv_fp8_async(q, len(codes.shape), codes.data_ptr(), plan.na_, plan.wa_, plan.pia_,
+                                   scales.data_ptr(), fibers_per_scale, b.data_ptr(), nb_, c.data_ptr(),
+                                   plan.nc_, wc_, plan.pic_, flags, _stream_ptr()))
     return c
 
 

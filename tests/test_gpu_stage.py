@@ -1,0 +1,58 @@
+"""The LDS-staged column products at the edges of their tiles against the FP64 oracle: one and many slabs per
+block, slabs of odd and even numbers of 16-byte vectors, ends that no vector fills, one and several rounds of
+outputs and contraction groups, unaligned bases, every storage type."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+NARROW = 8          # variant col_narrow
+
+# I, K, O
+SHAPES = [(2, 1, 1), (2, 2, 5), (3, 2, 4099), (3, 5, 1), (4, 16, 2049), (5, 7, 1200), (6, 4, 3001), (7, 129, 33),
+          (8, 2, 10000), (12, 341, 9), (16, 512, 3), (45, 13, 300), (64, 31, 40), (130, 63, 2), (1024, 8, 2), (4096, 2, 3)]
+
+
+@pytest.mark.parametrize("I,K,Ox", SHAPES)
+@pytest.mark.parametrize("dt", ["f32", "f64", "bf16", "fp8"])
+def test_staged_columns(ttvx, device, I, K, Ox, dt):
+    import torch
+    rng = np.random.default_rng(I * 1000 + K)
+    x = rng.uniform(-1, 1, (Ox, K, I))
+    b = rng.uniform(-1, 1, K)
+    real = np.float64 if dt == "f64" else np.float32
+    b = b.astype(real)
+    bd = torch.from_numpy(b).to(device)
+    scale = np.ones((Ox, I))
+    ttvx.set_selection(ttvx.SELECT_FORCED, NARROW)
+    try:
+        for off in (0, 1):          # elements past a 16-byte boundary
+            def place(values):
+                buf = torch.empty(values.size + off, dtype=torch.from_numpy(values[:0].ravel()).dtype, device=device)
+                buf[off:] = torch.from_numpy(values.ravel()).to(device)
+                return buf[off:].view(Ox, K, I)
+            if dt in ("f32", "f64"):
+                v = x.astype(real)
+                C = ttvx.ttv(2, place(v), bd)
+                v = v.astype(np.float64)
+            elif dt == "bf16":
+                bits = O.bf16_rne(x.astype(np.float32).ravel())
+                v = O.bf16_to_f32(bits).reshape(x.shape).astype(np.float64)
+                C = ttvx.ttv_bf16(2, place(bits.view(np.int16).reshape(x.shape)).view(torch.uint16), bd,
+                                  flags=ttvx.FLAG_KAHAN if off else 0)
+            else:
+                codes = rng.integers(0, 120, x.shape).astype(np.uint8)
+                v = O.e4m3_decode(codes.ravel()).reshape(x.shape).astype(np.float64)
+                fps = 3 if off else 1 + I // 2
+                s = rng.uniform(0.5, 2, -(-Ox * I // fps)).astype(np.float32)
+                scale = np.repeat(s.astype(np.float64), fps)[:Ox * I].reshape(Ox, I)
+                C = ttvx.ttv_fp8(2, place(codes), torch.from_numpy(s).to(device), fps, bd)
+            torch.cuda.synchronize()
+            terms = v * b.astype(np.float64)[None, :, None]
+            exact, mag = terms.sum(1) * scale, np.abs(terms).sum(1) * scale
+            # any order of K products and sums, then one scaling: (K + 2) roundings of the magnitudes
+            eps = 2.0 ** -53 if dt == "f64" else 2.0 ** -24
+            assert np.all(np.abs(C.cpu().numpy().astype(np.float64) - exact) <= (K + 2) * eps * mag + 1e-300)
+    finally:
+        ttvx.restore_default_selection()

@@ -322,6 +322,12 @@ struct Args {
 	int kpart;
 	// k_rows with LPR = ceil(K / VEC) lanes per row, not a power of two (rows_group, LPRC < 0)
 	int tight;
+	// k_stage: bytes from slab to slab in LDS, division by the lane vectors of a row and by the 16-byte vectors of a
+	// slab (itShift: log2 of the lanes along the outputs)
+	int pitch;
+	FastDiv by_i, by_slab;
+	int fps32;                // k_stage: outputs fit 31 bits, by_fps divides by fps
+	FastDiv by_fps;
 };
 
 // Range of work units [begin, end) with step of block blockIdx.x (lane offset added by callers)

@@ -13,6 +13,7 @@
 
 #include "../../include/ttvx.h"
 #include "mlp.hpp"
+#include "stage.hpp"
 
 // Waves per CU that the split row kernel aims for (its splits x row groups).  Measured on MI355X,
 // rows of 2^27-2^29 bytes, O = 2..100: 32 beats 8 and 16 by up to 30 % for 30 and more rows.
@@ -281,6 +282,45 @@ void configure_view(const Fold& f, const DType& dt, Config& cfg)
 		cfg.grid = static_cast<int>(blocks);
 	}
 }
+
+// col_narrow on slabs that are dense in A and fit a staging tile: k_stage (stage.hpp; faster than k_slab on all of them)
+bool configure_stage(const Fold& f, const DType& dt, Config& cfg)
+{
+	if(f.K * f.I > kStageBytes / dt.size) return false;
+	if(f.sAk != f.I || (f.O > 1 && f.sAo != f.K * f.I)) return false;
+	Args& P = cfg.args;
+	int64_t const slab = f.K * f.I * dt.size;
+	int const most = dt.size == 8 ? 2 : kStageMaxPV;
+	cfg.vec = f.I % 4 == 0 && most == 4 ? 4 : (f.I % 2 == 0 ? 2 : 1);
+	// slabs of an even number of 16-byte vectors start 16 bytes further apart in LDS, so that the lanes of a wave,
+	// which read the same position of neighbouring slabs, meet 16 different banks groups
+	P.pitch = static_cast<int>(slab % 32 == 0 && 2 * (slab + 16) <= kStageBytes ? slab + 16 : slab);
+	int64_t os = kStageBytes / P.pitch;
+	// small tensors: at least 4 blocks per CU before a block takes more slabs
+	os = std::min(os, std::max<int64_t>(1, f.O / (static_cast<int64_t>(cfg.cus) * 4)));
+	// every item starts on a 16-byte boundary of A's base where the tile has room for it
+	int64_t unit = 1;
+	while(unit < 16 && unit * slab % 16 != 0) unit *= 2;
+	if(os >= unit) os = os / unit * unit;
+	else if(unit * P.pitch <= kStageBytes) os = unit;
+	P.OS = static_cast<int>(os);
+	P.items = ceil_div(f.O, os);
+	if(P.items > kMaxLeanBlocks) return false;
+	int64_t const outputs = os * (f.I / cfg.vec);
+	int jl = 0;
+	while(jl < 8 && (int64_t{1} << jl) < outputs) ++jl;
+	P.itShift = jl;
+	P.by_i = fast_div(f.I / cfg.vec);
+	P.by_slab = fast_div(std::max<int64_t>(1, slab / 16));
+	P.kchunk = f.K;
+	cfg.ksplit = 1;
+	cfg.U = 1;
+	cfg.lean = LEAN_STAGE;
+	cfg.grid = static_cast<int>(P.items);
+	// the partial sums of the contraction groups take the same LDS afterwards
+	cfg.shmem = static_cast<std::size_t>(std::max<int64_t>(os * P.pitch, static_cast<int64_t>(kBlock) * cfg.vec * acc_size(dt)));
+	return true;
+}
 } // namespace
 
 bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus, unsigned flags, Config& cfg)
@@ -405,6 +445,8 @@ bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus,
 			P.items  = ceil_div(f.O, static_cast<int64_t>(P.OS) * cfg.U) * P.iTiles;
 		}
 		if(vb == V_COL_NARROW) {
+			if(fp64_final && dt.code != TTVX_F64) return false;      // no split partials in k_slab and k_stage
+			if(configure_stage(f, dt, cfg)) return true;
 			// k_slab: rows cut into chunks of IT <= kNarrowLanes vectors (a power of two), the block's
 			// other lanes along k (as many as K uses), OS slabs per block, one item per block
 			P.IT = static_cast<int>(std::min<int64_t>(int64_t{1} << ilog2(iv), kNarrowLanes));
@@ -422,7 +464,6 @@ bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus,
 			cfg.lean = LEAN_SLAB;
 			cfg.grid = static_cast<int>(std::max<int64_t>(1, P.items));
 			if(P.items > kMaxLeanBlocks) return false;               // one block per item
-			if(fp64_final && dt.code != TTVX_F64) return false;      // no split partials in k_slab
 			return true;
 		}
 		int64_t ksplit = 1;
@@ -698,6 +739,8 @@ int launch(const Fold& f, const DType& dt, const void* a, const void* b, void* c
 	} else if(cfg.kind != KIND_STRIDED) {
 		cfg.args.scales = scales;
 		cfg.args.fps    = fps > 0 ? fps : 1;
+		cfg.args.fps32  = cfg.lean == LEAN_STAGE && f.O * f.I < (int64_t{1} << 31) && cfg.args.fps < (int64_t{1} << 31) ? 1 : 0;
+		if(cfg.args.fps32) cfg.args.by_fps = fast_div(cfg.args.fps);
 	}
 
 	// 2- and 1-byte products whose vectors do not all start on a 4-byte boundary run the
@@ -711,11 +754,12 @@ int launch(const Fold& f, const DType& dt, const void* a, const void* b, void* c
 	uint64_t const a_low = reinterpret_cast<uintptr_t>(a) | static_cast<uint64_t>(f.sAo * dt.size);
 	bool const sub4 = dt.size < 4 && cfg.vec * dt.size >= 4 &&
 	                  ((cfg.kind == KIND_DOT && ((a_low | static_cast<uint64_t>(f.K * dt.size)) & 3u) != 0) ||
-	                   (cfg.kind == KIND_COL && cfg.lean != LEAN_SLAB && !cfg.args.one_step && cfg.args.IT >= 64 &&
+	                   (cfg.kind == KIND_COL && cfg.lean != LEAN_SLAB && cfg.lean != LEAN_STAGE && !cfg.args.one_step && cfg.args.IT >= 64 &&
 	                    ((a_low | static_cast<uint64_t>(f.sAk * dt.size)) & 3u) != 0));
 	if(injected(TTVX_FAULT_LAUNCH)) return hip_fail(hipErrorLaunchFailure, "kernel launch");
 	int rc = TTVX_OK;
-	switch(dt.code) {
+	if(cfg.lean == LEAN_STAGE) rc = launch_stage(cfg, dt.code, a, b, c, kahan, stream);
+	else switch(dt.code) {
 		case TTVX_F32:     rc = launch_f32 (cfg, a, b, c, kahan, stream); break;
 		case TTVX_F64:     rc = launch_f64 (cfg, a, b, c, kahan, stream); break;
 		case TTVX_BF16:    rc = sub4 ? launch_bf16_sub(cfg, a, b, c, kahan, stream) : launch_bf16(cfg, a, b, c, kahan, stream); break;

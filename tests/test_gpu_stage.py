@@ -1,4 +1,4 @@
-"""The LDS-staged column products at the edges of their tiles against the FP64 oracle: one and many slabs per
+"""The LDS-staged column and row products at the edges of their tiles against the FP64 oracle: one and many slabs per
 block, slabs of odd and even numbers of 16-byte vectors, ends that no vector fills, one and several rounds of
 outputs and contraction groups, unaligned bases, every storage type."""
 import numpy as np
@@ -7,16 +7,19 @@ import pytest
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
-NARROW = 8          # variant col_narrow
+NARROW, K_LANES = 8, 10          # variants col_narrow, col_k_lanes
 
 # I, K, O
 SHAPES = [(2, 1, 1), (2, 2, 5), (3, 2, 4099), (3, 5, 1), (4, 16, 2049), (5, 7, 1200), (6, 4, 3001), (7, 129, 33),
+          # rows: one and several lanes each, runs that end inside a word, one and many rounds, the longest
+          (1, 2, 40000), (1, 3, 7), (1, 5, 9001), (1, 16, 3000), (1, 31, 1030), (1, 129, 700), (1, 255, 300), (1, 512, 64),
+          (1, 1001, 37), (1, 1024, 9), (1, 2048, 6), (1, 4097, 5), (1, 8192, 4),
           (8, 2, 10000), (12, 341, 9), (16, 512, 3), (45, 13, 300), (64, 31, 40), (130, 63, 2), (1024, 8, 2), (4096, 2, 3)]
 
 
 @pytest.mark.parametrize("I,K,Ox", SHAPES)
 @pytest.mark.parametrize("dt", ["f32", "f64", "bf16", "fp8"])
-def test_staged_columns(ttvx, device, I, K, Ox, dt):
+def test_staged_products(ttvx, device, I, K, Ox, dt):
     import torch
     rng = np.random.default_rng(I * 1000 + K)
     x = rng.uniform(-1, 1, (Ox, K, I))
@@ -25,7 +28,7 @@ def test_staged_columns(ttvx, device, I, K, Ox, dt):
     b = b.astype(real)
     bd = torch.from_numpy(b).to(device)
     scale = np.ones((Ox, I))
-    ttvx.set_selection(ttvx.SELECT_FORCED, NARROW)
+    ttvx.set_selection(ttvx.SELECT_FORCED, NARROW if I > 1 else K_LANES)
     try:
         for off in (0, 1):          # elements past a 16-byte boundary
             def place(values):

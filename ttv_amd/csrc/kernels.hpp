@@ -322,6 +322,8 @@ struct Args {
 	int kpart;
 	// k_rows with LPR = ceil(K / VEC) lanes per row, not a power of two (rows_group, LPRC < 0)
 	int tight;
+	// k_stage_rows: swizzled LDS (stage_at)
+	int swz;
 	// k_stage: bytes from slab to slab in LDS, division by the lane vectors of a row and by the 16-byte vectors of a
 	// slab (itShift: log2 of the lanes along the outputs)
 	int pitch;

@@ -283,35 +283,41 @@ void configure_view(const Fold& f, const DType& dt, Config& cfg)
 	}
 }
 
-// col_narrow on slabs that are dense in A and fit a staging tile: k_stage (stage.hpp; faster than k_slab on all of them)
-bool configure_stage(const Fold& f, const DType& dt, Config& cfg)
+// Slabs (or rows) of `slab` bytes per staging tile and their pitch in LDS
+int64_t stage_tile(int64_t O, int64_t slab, int cus, Args& P)
 {
-	if(f.K * f.I > kStageBytes / dt.size) return false;
-	if(f.sAk != f.I || (f.O > 1 && f.sAo != f.K * f.I)) return false;
-	Args& P = cfg.args;
-	int64_t const slab = f.K * f.I * dt.size;
-	int const most = dt.size == 8 ? 2 : kStageMaxPV;
-	cfg.vec = f.I % 4 == 0 && most == 4 ? 4 : (f.I % 2 == 0 ? 2 : 1);
 	// slabs of an even number of 16-byte vectors start 16 bytes further apart in LDS, so that the lanes of a wave,
-	// which read the same position of neighbouring slabs, meet 16 different banks groups
+	// which read the same position of neighbouring slabs, spread over the banks
 	P.pitch = static_cast<int>(slab % 32 == 0 && 2 * (slab + 16) <= kStageBytes ? slab + 16 : slab);
 	int64_t os = kStageBytes / P.pitch;
 	// small tensors: at least 4 blocks per CU before a block takes more slabs
-	os = std::min(os, std::max<int64_t>(1, f.O / (static_cast<int64_t>(cfg.cus) * 4)));
+	os = std::min(os, std::max<int64_t>(1, O / (static_cast<int64_t>(cus) * 4)));
 	// every item starts on a 16-byte boundary of A's base where the tile has room for it
 	int64_t unit = 1;
 	while(unit < 16 && unit * slab % 16 != 0) unit *= 2;
 	if(os >= unit) os = os / unit * unit;
 	else if(unit * P.pitch <= kStageBytes) os = unit;
 	P.OS = static_cast<int>(os);
-	P.items = ceil_div(f.O, os);
+	P.items = ceil_div(O, os);
+	P.by_slab = fast_div(std::max<int64_t>(1, slab / 16));
+	return os;
+}
+
+// col_narrow on slabs that are dense in A and fit a staging tile: k_stage (stage.hpp; faster than k_slab on all of them)
+bool configure_stage(const Fold& f, const DType& dt, Config& cfg)
+{
+	if(f.K * f.I > kStageBytes / dt.size) return false;
+	if(f.sAk != f.I || (f.O > 1 && f.sAo != f.K * f.I)) return false;
+	Args& P = cfg.args;
+	int const most = dt.size == 8 ? 2 : kStageMaxPV;
+	cfg.vec = f.I % 4 == 0 && most == 4 ? 4 : (f.I % 2 == 0 ? 2 : 1);
+	int64_t const os = stage_tile(f.O, f.K * f.I * dt.size, cfg.cus, P);
 	if(P.items > kMaxLeanBlocks) return false;
 	int64_t const outputs = os * (f.I / cfg.vec);
 	int jl = 0;
 	while(jl < 8 && (int64_t{1} << jl) < outputs) ++jl;
 	P.itShift = jl;
 	P.by_i = fast_div(f.I / cfg.vec);
-	P.by_slab = fast_div(std::max<int64_t>(1, slab / 16));
 	P.kchunk = f.K;
 	cfg.ksplit = 1;
 	cfg.U = 1;
@@ -319,6 +325,34 @@ bool configure_stage(const Fold& f, const DType& dt, Config& cfg)
 	cfg.grid = static_cast<int>(P.items);
 	// the partial sums of the contraction groups take the same LDS afterwards
 	cfg.shmem = static_cast<std::size_t>(std::max<int64_t>(os * P.pitch, static_cast<int64_t>(kBlock) * cfg.vec * acc_size(dt)));
+	return true;
+}
+
+// col_k_lanes on dense rows of which a staging tile holds at least 4: k_stage_rows
+bool configure_stage_rows(const Fold& f, const DType& dt, Config& cfg)
+{
+	if(f.K > kStageBytes / 4 / dt.size || f.K < 2 || (f.O > 1 && f.sAo != f.K)) return false;
+	Args& P = cfg.args;
+	// rows of nearly a multiple of 256 bytes that carry no padding all start in the same banks: swizzled LDS
+	int64_t const row = f.K * dt.size, turn = row % 256;
+	P.swz = row % 32 != 0 && row > 300 && (turn < 16 || turn > 240) ? 1 : 0;
+	int64_t const os = stage_tile(f.O, row, cfg.cus, P);
+	if(P.items > kMaxLeanBlocks) return false;
+	int64_t const words = ceil_div(f.K * dt.size, dt.size == 8 ? 8 : 4);
+	// lanes per row: as many as the block has for its rows, with at least 4 words each
+	int gs = 0;
+	while(gs < 6 && (os << (gs + 1)) <= kBlock && words >> (gs + 3) > 0) ++gs;
+	P.itShift = gs;
+	P.kchunk = f.K;
+	cfg.vec = 1;
+	cfg.ksplit = 1;
+	cfg.U = P.swz ? 2 : 1;                // (the batched kernel's form)
+	cfg.lean = LEAN_STAGE_ROWS;
+	cfg.grid = static_cast<int>(P.items);
+	// a funnel-shifted word reads the one after it too; then b, when several lanes share a row
+	int64_t const tile = os * P.pitch + 16;
+	P.red = static_cast<int>(ceil_div(P.swz ? tile + tile / 256 * 16 + 16 : tile, 16) * 16);
+	cfg.shmem = static_cast<std::size_t>(P.red) + (gs > 0 ? static_cast<std::size_t>(f.K) * acc_size(dt) : 0);
 	return true;
 }
 } // namespace
@@ -486,8 +520,9 @@ bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus,
 		cfg.grid   = static_cast<int>(std::max<int64_t>(1, std::min(P.items, cap)));
 	} else if(v == V_COL_K_LANES) {
 		if(!dot_shape) return false;
-		// the column kernel on a row problem: lanes along k (scalar loads), summed across 64 lanes
 		cfg.kind = KIND_COL;
+		if(!fp64_final && configure_stage_rows(f, dt, cfg)) return true;
+		// the column kernel on a row problem: lanes along k (scalar loads), summed across 64 lanes
 		cfg.vec  = 1;
 		P.I = 1; P.IT = 1;
 		P.KS = static_cast<int>(std::min<int64_t>(64, pow2_ceil(f.K)));
@@ -739,7 +774,7 @@ int launch(const Fold& f, const DType& dt, const void* a, const void* b, void* c
 	} else if(cfg.kind != KIND_STRIDED) {
 		cfg.args.scales = scales;
 		cfg.args.fps    = fps > 0 ? fps : 1;
-		cfg.args.fps32  = cfg.lean == LEAN_STAGE && f.O * f.I < (int64_t{1} << 31) && cfg.args.fps < (int64_t{1} << 31) ? 1 : 0;
+		cfg.args.fps32  = (cfg.lean == LEAN_STAGE || cfg.lean == LEAN_STAGE_ROWS) && f.O * f.I < (int64_t{1} << 31) && cfg.args.fps < (int64_t{1} << 31) ? 1 : 0;
 		if(cfg.args.fps32) cfg.args.by_fps = fast_div(cfg.args.fps);
 	}
 
@@ -754,11 +789,11 @@ int launch(const Fold& f, const DType& dt, const void* a, const void* b, void* c
 	uint64_t const a_low = reinterpret_cast<uintptr_t>(a) | static_cast<uint64_t>(f.sAo * dt.size);
 	bool const sub4 = dt.size < 4 && cfg.vec * dt.size >= 4 &&
 	                  ((cfg.kind == KIND_DOT && ((a_low | static_cast<uint64_t>(f.K * dt.size)) & 3u) != 0) ||
-	                   (cfg.kind == KIND_COL && cfg.lean != LEAN_SLAB && cfg.lean != LEAN_STAGE && !cfg.args.one_step && cfg.args.IT >= 64 &&
+	                   (cfg.kind == KIND_COL && cfg.lean == LEAN_NONE && !cfg.args.one_step && cfg.args.IT >= 64 &&
 	                    ((a_low | static_cast<uint64_t>(f.sAk * dt.size)) & 3u) != 0));
 	if(injected(TTVX_FAULT_LAUNCH)) return hip_fail(hipErrorLaunchFailure, "kernel launch");
 	int rc = TTVX_OK;
-	if(cfg.lean == LEAN_STAGE) rc = launch_stage(cfg, dt.code, a, b, c, kahan, stream);
+	if(cfg.lean == LEAN_STAGE || cfg.lean == LEAN_STAGE_ROWS) rc = launch_stage(cfg, dt.code, a, b, c, kahan, stream);
 	else switch(dt.code) {
 		case TTVX_F32:     rc = launch_f32 (cfg, a, b, c, kahan, stream); break;
 		case TTVX_F64:     rc = launch_f64 (cfg, a, b, c, kahan, stream); break;

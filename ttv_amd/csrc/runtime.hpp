@@ -62,12 +62,13 @@ struct DType {
 DType dtype_of(int code);
 
 // Kernels of the one-wave-per-group regime (kernels.hpp): k_rows for rows of one vector per lane,
-// k_slab for col_narrow (k_stage, stage.hpp, where slabs are small); LEAN_NONE for the looping k_dot / k_col / k_strided.  Views that do not fold:
+// k_slab for col_narrow (k_stage, stage.hpp, where slabs are small), k_stage_rows for col_k_lanes on short rows;
+// LEAN_NONE for the looping k_dot / k_col / k_strided.  Views that do not fold:
 // k_view_cols / k_view_rows / k_view_long_rows (view.hpp).
 enum Lean {
 	LEAN_NONE = 0, LEAN_ROWS = 1, LEAN_SLAB = 2,
 	LEAN_VIEW_COLS = 3, LEAN_VIEW_ROWS = 4, LEAN_VIEW_LONG_ROWS = 5,
-	LEAN_STAGE = 6
+	LEAN_STAGE = 6, LEAN_STAGE_ROWS = 7
 };
 
 // Most blocks of kBlock threads in one launch (fewer than 2^32 work-items per grid dimension).
@@ -123,7 +124,7 @@ int launch_fp8 (const Config& cfg, const void* a, const void* b, void* c, bool k
 int launch_bf16_sub(const Config& cfg, const void* a, const void* b, void* c, bool kahan, hipStream_t s);
 int launch_fp8_sub (const Config& cfg, const void* a, const void* b, void* c, bool kahan, hipStream_t s);
 
-// LDS-staged column products of every storage type (stage.hip)
+// LDS-staged products of every storage type (stage.hip)
 int launch_stage(const Config& cfg, int dtype, const void* a, const void* b, void* c, bool kahan, hipStream_t s);
 
 // Device memory a caller provides for the split partial sums instead of the library's buffers.

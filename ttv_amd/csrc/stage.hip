@@ -1,4 +1,4 @@
-// Launches of the LDS-staged column products (stage.hpp) for every storage type.
+// Launches of the LDS-staged products (stage.hpp) for every storage type.
 #include "stage.hpp"
 
 #include "runtime.hpp"
@@ -21,10 +21,26 @@ void go(const Config& cfg, const void* a, const void* b, void* c, bool kahan, hi
 		                   static_cast<const Acc*>(b), c, cfg.args);
 }
 
+template<typename S, bool SWZ>
+void go_rows(const Config& cfg, const void* a, const void* b, void* c, bool kahan, hipStream_t s)
+{
+	using Acc = typename Traits<S>::acc;
+	dim3 const grid(static_cast<unsigned>(cfg.grid)), block(kBlock);
+	if(!std::is_same_v<Acc, double> && kahan)
+		hipLaunchKernelGGL((k_stage_rows<S, !std::is_same_v<Acc, double>, SWZ>), grid, block, cfg.shmem, s,
+		                   static_cast<const S*>(a), static_cast<const Acc*>(b), c, cfg.args);
+	else
+		hipLaunchKernelGGL((k_stage_rows<S, false, SWZ>), grid, block, cfg.shmem, s, static_cast<const S*>(a),
+		                   static_cast<const Acc*>(b), c, cfg.args);
+}
+
 template<typename S>
 void go_typed(const Config& cfg, const void* a, const void* b, void* c, bool kahan, hipStream_t s)
 {
-	if(cfg.vec == 4) {
+	if(cfg.lean == LEAN_STAGE_ROWS) {
+		if(cfg.args.swz) go_rows<S, true>(cfg, a, b, c, kahan, s);
+		else               go_rows<S, false>(cfg, a, b, c, kahan, s);
+	} else if(cfg.vec == 4) {
 		if constexpr(sizeof(S) < 8) go<S, 4>(cfg, a, b, c, kahan, s);
 	} else if(cfg.vec == 2) {
 		go<S, 2>(cfg, a, b, c, kahan, s);

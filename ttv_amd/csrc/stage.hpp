@@ -47,21 +47,16 @@ __device__ __forceinline__ void stage_read(const unsigned char* p, typename Trai
 	decode(v, x);
 }
 
-// Item: slabs [item*OS, item*OS + OS).  Thread t: outputs t % JL (+ JL, ...), contraction group t / JL of KG = 256 / JL
-// (JL = 1 << itShift lanes; several groups only when one round of lanes covers the item's outputs).
-template<typename S, int PV, bool KAHAN>
-__device__ __forceinline__ void stage_item(const S* __restrict__ A, const typename Traits<S>::acc* __restrict__ b,
-                                           void* __restrict__ C, const Args& P, int64_t item, unsigned char* lds)
+// SWZ: LDS holds byte a at a + 16 * (a / 256), so that rows of nearly a multiple of 256 bytes do not all start in
+// the same banks
+template<bool SWZ> __device__ __forceinline__ int stage_at(int a) { return SWZ ? a + ((a >> 8) << 4) : a; }
+
+// The block's `bytes` contiguous bytes from src into LDS, slabs of `slab` bytes P.pitch apart
+template<typename S, bool SWZ = false>
+__device__ __forceinline__ void stage_load(const unsigned char* src, int bytes, int slab, const Args& P, unsigned char* lds)
 {
-	using Acc = typename Traits<S>::acc;
 	constexpr int R = kStageBytes / (16 * kBlock);
 	int const t = static_cast<int>(threadIdx.x);
-	int64_t const o0 = item * P.OS;
-	int const slabs = static_cast<int>(P.O - o0 < P.OS ? P.O - o0 : P.OS);
-	int const K = static_cast<int>(P.K), I = static_cast<int>(P.I);
-	int const slab = K * I * static_cast<int>(sizeof(S));
-	int const bytes = slabs * slab;
-	const unsigned char* const src = reinterpret_cast<const unsigned char*>(A) + o0 * slab;
 	int const nv = bytes >> 4;
 	if(nv > 0) {
 		u32x4_b v[R];
@@ -77,7 +72,8 @@ __device__ __forceinline__ void stage_item(const S* __restrict__ A, const typena
 		for(int r = 0; r < R; ++r) {
 			int const idx = r * kBlock + t;
 			if(idx < nv) {
-				int const at = P.pitch == slab ? idx : idx + static_cast<int>(div_by(static_cast<uint32_t>(idx), P.by_slab));
+				int const at = SWZ ? idx + (idx >> 4)
+				                   : (P.pitch == slab ? idx : idx + static_cast<int>(div_by(static_cast<uint32_t>(idx), P.by_slab)));
 				reinterpret_cast<u32x4*>(lds)[at] = v[r];
 			}
 		}
@@ -85,7 +81,24 @@ __device__ __forceinline__ void stage_item(const S* __restrict__ A, const typena
 	// the end of the last block's run (no padding there: a padded slab is whole vectors)
 #pragma unroll 1
 	for(int e = nv * 16 + t * static_cast<int>(sizeof(S)); e < bytes; e += kBlock * static_cast<int>(sizeof(S)))
-		*reinterpret_cast<S*>(lds + e) = *reinterpret_cast<const S*>(src + e);
+		*reinterpret_cast<S*>(lds + stage_at<SWZ>(e)) = *reinterpret_cast<const S*>(src + e);
+}
+
+// Item: slabs [item*OS, item*OS + OS).  Thread t: outputs t % JL (+ JL, ...), contraction group t / JL of KG = 256 / JL
+// (JL = 1 << itShift lanes; several groups only when one round of lanes covers the item's outputs).
+template<typename S, int PV, bool KAHAN>
+__device__ __forceinline__ void stage_item(const S* __restrict__ A, const typename Traits<S>::acc* __restrict__ b,
+                                           void* __restrict__ C, const Args& P, int64_t item, unsigned char* lds)
+{
+	using Acc = typename Traits<S>::acc;
+	int const t = static_cast<int>(threadIdx.x);
+	int64_t const o0 = item * P.OS;
+	int const slabs = static_cast<int>(P.O - o0 < P.OS ? P.O - o0 : P.OS);
+	int const K = static_cast<int>(P.K), I = static_cast<int>(P.I);
+	int const slab = K * I * static_cast<int>(sizeof(S));
+	int const bytes = slabs * slab;
+	const unsigned char* const src = reinterpret_cast<const unsigned char*>(A) + o0 * slab;
+	stage_load<S>(src, bytes, slab, P, lds);
 	__syncthreads();
 
 	int const JL = 1 << P.itShift, KG = kBlock >> P.itShift;
@@ -183,6 +196,138 @@ __device__ __forceinline__ void stage_item(const S* __restrict__ A, const typena
 		}
 		if(KG > 1) return;
 	}
+}
+
+// MI355X, 256 MiB, GB/s of k_stage_rows against the best direct row kernel (k_rows, k_dot):
+//   row length   FP64          BF16          FP8
+//   33           6061 / 5627   5962 / 4471   4775 / 3096
+//   129          6292 / 3437   5300 / 4344   5743 / 3273
+//   255          6126 / 4356   5011 / 4711   4536 / 4334
+//   513          5576 / 4390   4471 / 3213   4194 / 2955
+// Rows of whole 16-byte vectors of the 4-, 2- and 1-byte types stay with k_rows (FP8 rows of 128: 5678 / 5797), and
+// the swizzle is for rows whose starts would collide (FP8 rows of 511 without it 2.8 TB/s).
+// Rows (q fastest) in the same way: item = rows [item*OS, item*OS + OS), G = 1 << itShift neighbouring lanes per row,
+// which take its words (of 4 bytes; 8 for FP64) in turn.  Words are read from the aligned ones that hold them, so
+// rows of 2- and 1-byte storage may start anywhere.
+template<typename S, bool KAHAN, bool SWZ>
+__device__ __forceinline__ void stage_rows_item(const S* __restrict__ A, const typename Traits<S>::acc* __restrict__ b,
+                                                void* __restrict__ C, const Args& P, int64_t item, unsigned char* lds)
+{
+	using Acc = typename Traits<S>::acc;
+	constexpr int WB = sizeof(S) == 8 ? 8 : 4;                        // bytes of a word
+	constexpr int E = WB / static_cast<int>(sizeof(S));               // elements of a word
+	int const t = static_cast<int>(threadIdx.x);
+	int64_t const o0 = item * P.OS;
+	int const rows = static_cast<int>(P.O - o0 < P.OS ? P.O - o0 : P.OS);
+	int const K = static_cast<int>(P.K);
+	int const row = K * static_cast<int>(sizeof(S));
+	int const G = 1 << P.itShift;
+	// with several lanes per row b comes from LDS too (through the vector cache it took as long as A: BF16 rows of
+	// 256 4.3 TB/s)
+	Acc* const lb = reinterpret_cast<Acc*>(lds + P.red);
+	if(G > 1)
+		for(int k = t; k < K; k += kBlock) lb[k] = b[k];
+	stage_load<S, SWZ>(reinterpret_cast<const unsigned char*>(A) + o0 * row, rows * row, row, P, lds);
+	__syncthreads();
+
+	int const g = t & (G - 1);
+	int const words = K / E;                                          // whole words of a row
+#pragma unroll 1
+	for(int r0 = 0; r0 < rows; r0 += kBlock >> P.itShift) {
+		int const r = r0 + (t >> P.itShift);
+		bool const live = r < rows;
+		int const at = (live ? r : 0) * P.pitch;
+		int const at0 = at & ~(WB - 1);                               // the word at or below the row's first element
+		uint32_t const m = static_cast<uint32_t>(at & 3);
+		Sum<Acc, KAHAN> acc;
+		// N words w, w + step, ... of the row into x; those of 2- and 1-byte storage are funnel-shifted from the two
+		// aligned words that hold them
+		auto words_at = [&](auto n_, int w, int step, auto& x) {
+			constexpr int N = decltype(n_)::value;
+			if constexpr(sizeof(S) == 8) {
+#pragma unroll
+				for(int u = 0; u < N; ++u) x[u] = *reinterpret_cast<const double*>(lds + stage_at<SWZ>(at0 + 8 * (w + u * step)));
+			} else if constexpr(sizeof(S) == 4) {
+#pragma unroll
+				for(int u = 0; u < N; ++u) x[u] = *reinterpret_cast<const float*>(lds + stage_at<SWZ>(at0 + 4 * (w + u * step)));
+			} else {
+				uint32_t lo[N], hi[N];
+#pragma unroll
+				for(int u = 0; u < N; ++u) {
+					int const a = at0 + 4 * (w + u * step);
+					lo[u] = *reinterpret_cast<const uint32_t*>(lds + stage_at<SWZ>(a));
+					hi[u] = *reinterpret_cast<const uint32_t*>(lds + stage_at<SWZ>(a + 4));
+				}
+#pragma unroll
+				for(int u = 0; u < N; ++u) {
+					Vec<S, E> v;
+					v.w[0] = __builtin_amdgcn_alignbyte(hi[u], lo[u], m);
+					Acc y[E];
+					decode(v, y);
+#pragma unroll
+					for(int e = 0; e < E; ++e) x[u * E + e] = y[e];
+				}
+			}
+		};
+		auto run = [&](auto lds_b, const Acc* bp, int w, int step) {
+			constexpr bool kLds = decltype(lds_b)::value;
+			int left = w < words ? (words - 1 - w) / step + 1 : 0;
+			auto round = [&](auto n_) {
+				constexpr int N = decltype(n_)::value;
+				Acc x[N * E], bv[N * E];
+#pragma unroll
+				for(int u = 0; u < N; ++u) {
+					struct alignas(E * sizeof(Acc)) Word { Acc v[E]; };
+					if constexpr(kLds) {
+						Word const q = *reinterpret_cast<const Word*>(bp + u * step * E);
+#pragma unroll
+						for(int e = 0; e < E; ++e) bv[u * E + e] = q.v[e];
+					} else {
+#pragma unroll
+						for(int e = 0; e < E; ++e) bv[u * E + e] = bp[u * step * E + e];
+					}
+				}
+				words_at(n_, w, step, x);
+#pragma unroll
+				for(int u = 0; u < N * E; ++u) acc.fma(x[u], bv[u]);
+				w += N * step;
+				bp += N * step * E;
+				left -= N;
+			};
+#pragma unroll 1
+			while(left >= 8) round(std::integral_constant<int, 8>{});
+			if(left >= 4) round(std::integral_constant<int, 4>{});
+			if(left >= 2) round(std::integral_constant<int, 2>{});
+			if(left >= 1) round(std::integral_constant<int, 1>{});
+		};
+		if(G == 1) run(std::false_type{}, b, 0, 1);   // one k for a whole wave: b through the scalar cache
+		else       run(std::true_type{}, lb + g * E, g, G);
+		if constexpr(E > 1) {
+			// the last elements of a row whose length a word does not divide
+			if(g == 0)
+				for(int k = words * E; k < K; ++k) {
+					Acc x[1];
+					stage_read<S, 1>(lds + stage_at<SWZ>(at + k * static_cast<int>(sizeof(S))), x);
+					acc.fma(x[0], b[k]);
+				}
+		}
+		Acc v = acc.value();
+		for(int d = G >> 1; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+		if(live && g == 0) {
+			int64_t const o = o0 + r;
+			if constexpr(kScaled<S>)
+				if(P.scales != nullptr) v *= P.fps32 ? P.scales[div_by(static_cast<uint32_t>(o), P.by_fps)] : P.scales[o / P.fps];
+			static_cast<Acc*>(C)[o * P.sCo] = v;
+		}
+	}
+}
+
+template<typename S, bool KAHAN, bool SWZ>
+__global__ __launch_bounds__(kBlock, 5) void k_stage_rows(const S* __restrict__ A, const typename Traits<S>::acc* __restrict__ b,
+                                                          void* __restrict__ C, Args P)
+{
+	extern __shared__ __attribute__((aligned(16))) unsigned char stage_lds[];
+	stage_rows_item<S, KAHAN, SWZ>(A, b, C, P, blockIdx.x, stage_lds);
 }
 
 // (at most 96 registers: 5 waves per SIMD, as many as the LDS leaves room for)

@@ -59,3 +59,56 @@ def test_staged_products(ttvx, device, I, K, Ox, dt):
             assert np.all(np.abs(C.cpu().numpy().astype(np.float64) - exact) <= (K + 2) * eps * mag + 1e-300)
     finally:
         ttvx.restore_default_selection()
+
+
+SPLIT_COL, SPLIT_DOT = 9, 4          # variants col_split, dot_split
+
+# I, K, O: FP64 chunks of rows (one and several per block, split and unsplit, odd rows, few and many lane vectors);
+# long rows (2 and 4 vectors per lane, 1, 2 and 4 waves along the row, odd numbers of rows, several pieces per wave)
+LONG = [(2, 20000, 3), (3, 11003, 5), (16, 4100, 1), (45, 900, 7), (64, 2100, 2), (255, 131, 9), (100, 3000, 2),
+        (1024, 67, 3), (513, 300, 1), (7, 1 << 20, 1),
+        (1, 1025, 3), (1, 2049, 6), (1, 2500, 1001), (1, 4096, 37), (1, 5003, 258), (1, 16385, 5), (1, 100003, 3),
+        (1, 300001, 64)]
+
+
+@pytest.mark.parametrize("I,K,Ox", LONG)
+@pytest.mark.parametrize("dt", ["f32", "f64", "bf16", "fp8"])
+def test_long_contractions(ttvx, device, I, K, Ox, dt):
+    import torch
+    rng = np.random.default_rng(I * 7 + K)
+    x = rng.uniform(-1, 1, (Ox, K, I)).astype(np.float64 if dt == "f64" else np.float32)
+    b = rng.uniform(-1, 1, K).astype(x.dtype)
+    bd = torch.from_numpy(b).to(device)
+    scale = np.ones((Ox, I))
+    ttvx.set_selection(ttvx.SELECT_FORCED, SPLIT_COL if I > 1 else SPLIT_DOT)
+    try:
+        for off, flags in ((0, 0), (1, 0), (0, ttvx.FLAG_FP64_FINAL)):
+            if flags and I > 1:
+                continue        # not every one of these shapes splits, and the rule's FP8 pick has no FP64 partial sums
+            def place(values):
+                buf = torch.empty(values.size + off, dtype=torch.from_numpy(values[:0].ravel()).dtype, device=device)
+                buf[off:] = torch.from_numpy(values.ravel()).to(device)
+                return buf[off:].view(Ox, K, I)
+            if dt in ("f32", "f64"):
+                v = x.astype(np.float64)
+                C = ttvx.ttv(2, place(x), bd, flags=flags)
+            elif dt == "bf16":
+                bits = O.bf16_rne(x.ravel())
+                v = O.bf16_to_f32(bits).reshape(x.shape).astype(np.float64)
+                C = ttvx.ttv_bf16(2, place(bits.view(np.int16).reshape(x.shape)).view(torch.uint16), bd,
+                                  flags=flags | (ttvx.FLAG_KAHAN if off else 0))
+            else:
+                codes = rng.integers(0, 120, x.shape).astype(np.uint8)
+                v = O.e4m3_decode(codes.ravel()).reshape(x.shape).astype(np.float64)
+                fps = 1 + I // 2
+                s = rng.uniform(0.5, 2, -(-Ox * I // fps)).astype(np.float32)
+                scale = np.repeat(s.astype(np.float64), fps)[:Ox * I].reshape(Ox, I)
+                C = ttvx.ttv_fp8(2, place(codes), torch.from_numpy(s).to(device), fps, bd, flags=flags)
+            torch.cuda.synchronize()
+            terms = v * b.astype(np.float64)[None, :, None]
+            exact, mag = terms.sum(1) * scale, np.abs(terms).sum(1) * scale
+            # no output sums more than K / 64 terms in one chain: far inside (K / 8 + 64) roundings of the magnitudes
+            eps = 2.0 ** -53 if dt == "f64" else 2.0 ** -24
+            assert np.all(np.abs(C.cpu().numpy().astype(np.float64) - exact) <= (K / 8 + 64) * eps * mag + 1e-300)
+    finally:
+        ttvx.restore_default_selection()

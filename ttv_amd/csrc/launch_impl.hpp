@@ -5,6 +5,7 @@
 
 #include <algorithm>
 
+#include "longrows.hpp"
 #include "runtime.hpp"
 #include "view.hpp"
 
@@ -64,6 +65,15 @@ int launch_vec(const Config& cfg, const S* A, const typename Traits<S>::acc* B, 
 			return TTVX_OK;
 		}
 		return fail(TTVX_ERR_UNSUPPORTED, "ttvx: realigned loads for row and column products only");
+	}
+	if(cfg.lean == LEAN_LONG_ROWS) {
+		if constexpr(VEC == Traits<S>::vmax) {
+			dim3 const g2(static_cast<unsigned>(cfg.grid), static_cast<unsigned>(cfg.ksplit));
+			if(cfg.U == 2) hipLaunchKernelGGL((k_long_rows<S, VEC, 2, KH>), g2, block, 0, s, A, B, C, cfg.args);
+			else           hipLaunchKernelGGL((k_long_rows<S, VEC, 4, KH>), g2, block, 0, s, A, B, C, cfg.args);
+			return TTVX_OK;
+		}
+		return fail(TTVX_ERR_UNSUPPORTED, "ttvx: long rows take full-width vectors");
 	}
 	if(cfg.lean == LEAN_ROWS) {
 		switch(cfg.U) {

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "../../include/ttvx.h"
+#include "longrows.hpp"
 #include "mlp.hpp"
 #include "stage.hpp"
 
@@ -283,6 +284,40 @@ void configure_view(const Fold& f, const DType& dt, Config& cfg)
 	}
 }
 
+// dot_split on three and more rows of more than one vector per lane: k_long_rows (longrows.hpp)
+bool configure_long_rows(const Fold& f, const DType& dt, Config& cfg)
+{
+	int64_t const vsteps = ceil_div(f.K, cfg.vec);
+	// one or two rows: no b to share, the looping kernel streams both operands
+	if(cfg.vec != dt.vmax || vsteps <= 64 || f.O < 3) return false;
+	Args& P = cfg.args;
+	int const n = vsteps <= 128 ? 2 : 4;
+	int64_t const piece = long_piece(cfg.vec, n);
+	int64_t const pieces = ceil_div(f.K, piece);
+	// waves of a block along the row: as many as leave at most an eighth of them without a piece
+	P.KS = 4;
+	while(P.KS > 1 && 8 * ceil_div(pieces, P.KS) * P.KS > 9 * pieces) P.KS >>= 1;
+	// waves for 16 per CU, but at least 8 rows (4- and 8-byte storage: 4) for each read of b
+	int64_t const waves = static_cast<int64_t>(cfg.cus) * 16;
+	int64_t const least = dt.size >= 4 ? 4 : 8;
+	int64_t rows = std::min<int64_t>({f.O, kLongMaxRows, std::max(least, f.O * pieces / waves)});
+	rows = ceil_div(f.O, ceil_div(f.O, rows));                   // even shares
+	int64_t const per_block = rows * (kBlock / 64 / P.KS);
+	int64_t const gx = ceil_div(f.O, per_block);
+	if(gx > kMaxLeanBlocks / 4) return false;
+	// more pieces per wave once there are waves enough, so that the partial sums stay few
+	int64_t const kiter = std::max<int64_t>({1, pieces * ceil_div(f.O, rows) / (2 * waves), ceil_div(pieces, 4096 * P.KS)});
+	P.OS = static_cast<int>(rows);
+	P.kiter = static_cast<int>(std::min<int64_t>(kiter, 1 << 20));
+	P.kchunk = P.kiter * P.KS * piece;
+	cfg.ksplit = static_cast<int>(ceil_div(f.K, P.kchunk));
+	if(cfg.ksplit > 4096) return false;
+	cfg.U = n;
+	cfg.lean = LEAN_LONG_ROWS;
+	cfg.grid = static_cast<int>(gx);
+	return true;
+}
+
 // Slabs (or rows) of `slab` bytes per staging tile and their pitch in LDS
 int64_t stage_tile(int64_t O, int64_t slab, int cus, Args& P)
 {
@@ -310,14 +345,15 @@ bool configure_stage(const Fold& f, const DType& dt, Config& cfg)
 	if(f.sAk != f.I || (f.O > 1 && f.sAo != f.K * f.I)) return false;
 	Args& P = cfg.args;
 	int const most = dt.size == 8 ? 2 : kStageMaxPV;
-	cfg.vec = f.I % 4 == 0 && most == 4 ? 4 : (f.I % 2 == 0 ? 2 : 1);
+	int const vec = f.I % 4 == 0 && most == 4 ? 4 : (f.I % 2 == 0 ? 2 : 1);
 	int64_t const os = stage_tile(f.O, f.K * f.I * dt.size, cfg.cus, P);
 	if(P.items > kMaxLeanBlocks) return false;
-	int64_t const outputs = os * (f.I / cfg.vec);
+	int64_t const outputs = os * (f.I / vec);
 	int jl = 0;
 	while(jl < 8 && (int64_t{1} << jl) < outputs) ++jl;
 	P.itShift = jl;
-	P.by_i = fast_div(f.I / cfg.vec);
+	P.by_i = fast_div(f.I / vec);
+	cfg.vec = vec;
 	P.kchunk = f.K;
 	cfg.ksplit = 1;
 	cfg.U = 1;
@@ -402,6 +438,10 @@ bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus,
 		P.groups = ceil_div(f.O, rpw * cfg.U);
 		int64_t const waves_wanted = static_cast<int64_t>(std::max(cus, 1)) * 4 * 4;
 		int64_t ksplit = 1;
+		if(v == V_DOT_SPLIT && configure_long_rows(f, dt, cfg)) {
+			if(fp64_final && dt.code != TTVX_F64) P.part64 = 1;
+			return true;
+		}
 		if(v == V_DOT_SPLIT) {
 			if(P.groups >= waves_wanted || vsteps < 4 * P.LPR) return false;  // nothing to gain
 			// up to 4096 splits: a few long rows (O = 2, K = 2^27) still fill the GPU with waves
@@ -735,6 +775,28 @@ int partial_buffer(int device, hipStream_t stream, std::size_t bytes, void** out
 	return TTVX_OK;
 }
 
+namespace
+{
+// whether the stream's partials buffer already holds `bytes`
+bool partial_buffer_ready(int device, hipStream_t stream, std::size_t bytes)
+{
+	PartialBuffers& pb = g_partials[device & 63];
+	std::lock_guard<std::mutex> lock(pb.mutex);
+	auto const it = pb.by_stream.find(stream);
+	return it != pb.by_stream.end() && it->second.second >= bytes;
+}
+
+bool capturing(hipStream_t stream)
+{
+	hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+	if(hipStreamIsCapturing(stream, &st) != hipSuccess) {
+		(void)hipGetLastError();
+		return true;      // the legacy stream while another captures: no allocation either
+	}
+	return st != hipStreamCaptureStatusNone;
+}
+} // namespace
+
 int launch(const Fold& f, const DType& dt, const void* a, const void* b, void* c,
            const float* scales, int64_t fps, unsigned flags, int variant, hipStream_t stream, const Scratch* scratch)
 {
@@ -747,6 +809,14 @@ int launch(const Fold& f, const DType& dt, const void* a, const void* b, void* c
 		variant = heuristic_variant(f, dt, a_addr, flags);
 		if(!configure(variant, f, dt, a_addr, di.cus, flags, cfg))
 			return fail(TTVX_ERR_UNSUPPORTED, "ttvx: no kernel variant can run this problem");
+	}
+	// products that one pass can do as well do not split where their partial sums exceed the caller's scratch or
+	// would need an allocation that a capture forbids
+	if(cfg.lean == LEAN_LONG_ROWS && cfg.ksplit > 1) {
+		std::size_t const bytes = static_cast<std::size_t>(cfg.ksplit) * static_cast<std::size_t>(f.O * f.I) *
+		                          (cfg.args.part64 ? 8 : acc_size(dt));
+		if(scratch != nullptr ? bytes > scratch->bytes : !partial_buffer_ready(di.id, stream, bytes) && capturing(stream))
+			configure(V_DOT_U2, f, dt, a_addr, di.cus, flags, cfg);
 	}
 	bool const kahan = (flags & TTVX_FLAG_KAHAN) != 0;
 	set_output_stores(cfg, f, dt, reinterpret_cast<uintptr_t>(c));

@@ -364,6 +364,39 @@ bool configure_stage(const Fold& f, const DType& dt, Config& cfg)
 	return true;
 }
 
+// col_split on dense FP64 slabs of more than a staging tile with rows that a block's lanes hold: k_stage_chunks
+bool configure_stage_chunks(const Fold& f, const DType& dt, Config& cfg)
+{
+	int64_t const row = f.I * dt.size;
+	// FP64 only: the direct column tiles reach 3.8-5.3 TB/s there (256 MiB, rows of 45 to 256, contractions of 300 and
+	// 1000) against 4.9-5.9 here.  For the narrower types they reach 5.3-6.3 at whole vectors, which this loop of
+	// loads and sums in turn does not, and very long contractions of any type split better there.
+	if(dt.size != 8 || f.K > 8192) return false;
+	if(f.K * row <= kStageBytes || f.O > kMaxLeanBlocks) return false;
+	if(f.sAk != f.I || (f.O > 1 && f.sAo != f.K * f.I)) return false;
+	Args& P = cfg.args;
+	int const vec = f.I % 2 == 0 ? 2 : 1;
+	int64_t const n = f.I / vec;
+	if(n > kBlock) return false;             // one lane vector of outputs per thread
+	int jl = 0;
+	while(jl < 8 && (int64_t{1} << jl) < n) ++jl;
+	P.itShift = jl;
+	P.OS = static_cast<int>(kStageBytes / row);
+	int64_t const chunks = ceil_div(f.K, P.OS);
+	// splits while the slabs leave the chip short of its 5 blocks per CU, each with at least two chunks
+	int64_t const want = static_cast<int64_t>(cfg.cus) * 5;
+	int64_t const ksplit = std::max<int64_t>(1, std::min<int64_t>({ceil_div(want, f.O), chunks / 2, 4096}));
+	P.kchunk = ceil_div(chunks, ksplit) * P.OS;
+	cfg.ksplit = static_cast<int>(ceil_div(f.K, P.kchunk));
+	cfg.vec = vec;
+	P.pitch = kStageBytes;                   // b of a chunk behind the tile, when a wave spans several rows
+	cfg.U = 1;
+	cfg.lean = LEAN_STAGE_CHUNKS;
+	cfg.grid = static_cast<int>(f.O);
+	cfg.shmem = static_cast<std::size_t>(kStageBytes) + (jl < 6 ? static_cast<std::size_t>(P.OS) * acc_size(dt) : 0);
+	return true;
+}
+
 // col_k_lanes on dense rows of which a staging tile holds at least 4: k_stage_rows
 bool configure_stage_rows(const Fold& f, const DType& dt, Config& cfg)
 {
@@ -517,6 +550,10 @@ bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus,
 		} else {
 			P.iTiles = ceil_div(iv, P.IT);
 			P.items  = ceil_div(f.O, static_cast<int64_t>(P.OS) * cfg.U) * P.iTiles;
+		}
+		if(vb == V_COL_SPLIT && configure_stage_chunks(f, dt, cfg)) {
+			if(fp64_final && dt.code != TTVX_F64) P.part64 = 1;
+			return true;
 		}
 		if(vb == V_COL_NARROW) {
 			if(fp64_final && dt.code != TTVX_F64) return false;      // no split partials in k_slab and k_stage
@@ -812,11 +849,11 @@ int launch(const Fold& f, const DType& dt, const void* a, const void* b, void* c
 	}
 	// products that one pass can do as well do not split where their partial sums exceed the caller's scratch or
 	// would need an allocation that a capture forbids
-	if(cfg.lean == LEAN_LONG_ROWS && cfg.ksplit > 1) {
+	if((cfg.lean == LEAN_LONG_ROWS || cfg.lean == LEAN_STAGE_CHUNKS) && cfg.ksplit > 1) {
 		std::size_t const bytes = static_cast<std::size_t>(cfg.ksplit) * static_cast<std::size_t>(f.O * f.I) *
 		                          (cfg.args.part64 ? 8 : acc_size(dt));
 		if(scratch != nullptr ? bytes > scratch->bytes : !partial_buffer_ready(di.id, stream, bytes) && capturing(stream))
-			configure(V_DOT_U2, f, dt, a_addr, di.cus, flags, cfg);
+			configure(cfg.lean == LEAN_LONG_ROWS ? V_DOT_U2 : V_COL_U1, f, dt, a_addr, di.cus, flags, cfg);
 	}
 	bool const kahan = (flags & TTVX_FLAG_KAHAN) != 0;
 	set_output_stores(cfg, f, dt, reinterpret_cast<uintptr_t>(c));
@@ -863,7 +900,7 @@ int launch(const Fold& f, const DType& dt, const void* a, const void* b, void* c
 	                    ((a_low | static_cast<uint64_t>(f.sAk * dt.size)) & 3u) != 0));
 	if(injected(TTVX_FAULT_LAUNCH)) return hip_fail(hipErrorLaunchFailure, "kernel launch");
 	int rc = TTVX_OK;
-	if(cfg.lean == LEAN_STAGE || cfg.lean == LEAN_STAGE_ROWS) rc = launch_stage(cfg, dt.code, a, b, c, kahan, stream);
+	if(cfg.lean == LEAN_STAGE || cfg.lean == LEAN_STAGE_ROWS || cfg.lean == LEAN_STAGE_CHUNKS) rc = launch_stage(cfg, dt.code, a, b, c, kahan, stream);
 	else switch(dt.code) {
 		case TTVX_F32:     rc = launch_f32 (cfg, a, b, c, kahan, stream); break;
 		case TTVX_F64:     rc = launch_f64 (cfg, a, b, c, kahan, stream); break;

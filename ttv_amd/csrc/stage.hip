@@ -21,6 +21,13 @@ void go(const Config& cfg, const void* a, const void* b, void* c, bool kahan, hi
 		                   static_cast<const Acc*>(b), c, cfg.args);
 }
 
+template<int PV>
+void go_chunks(const Config& cfg, const void* a, const void* b, void* c, hipStream_t s)
+{
+	hipLaunchKernelGGL((k_stage_chunks<PV>), dim3(static_cast<unsigned>(cfg.grid), static_cast<unsigned>(cfg.ksplit)),
+	                   dim3(kBlock), cfg.shmem, s, static_cast<const double*>(a), static_cast<const double*>(b), c, cfg.args);
+}
+
 template<typename S, bool SWZ>
 void go_rows(const Config& cfg, const void* a, const void* b, void* c, bool kahan, hipStream_t s)
 {
@@ -40,6 +47,11 @@ void go_typed(const Config& cfg, const void* a, const void* b, void* c, bool kah
 	if(cfg.lean == LEAN_STAGE_ROWS) {
 		if(cfg.args.swz) go_rows<S, true>(cfg, a, b, c, kahan, s);
 		else               go_rows<S, false>(cfg, a, b, c, kahan, s);
+	} else if(cfg.lean == LEAN_STAGE_CHUNKS) {
+		if constexpr(sizeof(S) == 8) {
+			if(cfg.vec == 2) go_chunks<2>(cfg, a, b, c, s);
+			else             go_chunks<1>(cfg, a, b, c, s);
+		}
 	} else if(cfg.vec == 4) {
 		if constexpr(sizeof(S) < 8) go<S, 4>(cfg, a, b, c, kahan, s);
 	} else if(cfg.vec == 2) {

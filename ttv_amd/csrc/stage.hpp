@@ -330,6 +330,87 @@ __global__ __launch_bounds__(kBlock, 5) void k_stage_rows(const S* __restrict__ 
 	stage_rows_item<S, KAHAN, SWZ>(A, b, C, P, blockIdx.x, stage_lds);
 }
 
+// FP64 slabs that no tile holds, in chunks of OS whole rows (dense slabs: a chunk is one contiguous run, whatever the
+// row length).  Block (x, y): slab x, contraction rows [y*kchunk, (y+1)*kchunk).  A lane keeps its outputs (vector
+// t % JL) over all chunks; the 5 blocks of a CU overlap each other's loads and sums.
+// MI355X, 256 MiB, GB/s against the best direct column tile, contractions of 300 and 1000: rows of 64 5879 / 5280,
+// 5258 / 5321; of 100 5065 / 4346, 5180 / 3813; of 255 5436 / 4556, 5071 / 4042; of 256 5045 / 5173, 4587 / 5189.
+template<int PV>
+__global__ __launch_bounds__(kBlock, 5) void k_stage_chunks(const double* __restrict__ A, const double* __restrict__ b,
+                                                            void* __restrict__ C, Args P)
+{
+	extern __shared__ __attribute__((aligned(16))) unsigned char stage_lds[];
+	unsigned char* const lds = stage_lds;
+	constexpr int SZ = 8;
+	int const t = static_cast<int>(threadIdx.x);
+	int64_t const o = blockIdx.x;
+	int const I = static_cast<int>(P.I), row = I * SZ;
+	int64_t const kb = static_cast<int64_t>(blockIdx.y) * P.kchunk;
+	int64_t const ke = kb + P.kchunk < P.K ? kb + P.kchunk : P.K;
+	double* const lb = reinterpret_cast<double*>(lds + P.pitch);      // the chunk's b (lanes of a wave on several rows)
+	int const JL = 1 << P.itShift, KG = kBlock >> P.itShift;
+	int const jl = t & (JL - 1), kg = t >> P.itShift;
+	int const n = I / PV;
+	int const j = jl < n ? jl : n - 1;       // spare lanes repeat the last output and store nothing
+	int const step = KG * row;
+	bool const uniform = JL >= 64;           // one k for a whole wave: b through the scalar cache
+	Sum<double, false> acc[PV];
+	for(int64_t k = kb; k < ke; k += P.OS) {
+		int const rows = static_cast<int>(ke - k < P.OS ? ke - k : P.OS);
+		stage_load<double>(reinterpret_cast<const unsigned char*>(A + (o * P.K + k) * I), rows * row, P.pitch, P, lds);
+		if(!uniform)
+			for(int q = t; q < rows; q += kBlock) lb[q] = b[k + q];
+		__syncthreads();
+		const unsigned char* p = lds + j * PV * SZ + kg * row;
+		auto sum = [&](const double* bp) {
+			int left = kg < rows ? (rows - 1 - kg) / KG + 1 : 0;
+			auto round = [&](auto n_) {
+				constexpr int N = decltype(n_)::value;
+				double x[N][PV];
+#pragma unroll
+				for(int u = 0; u < N; ++u) stage_read<double, PV>(p + u * step, x[u]);
+#pragma unroll
+				for(int u = 0; u < N; ++u)
+#pragma unroll
+					for(int e = 0; e < PV; ++e) acc[e].fma(x[u][e], bp[u * KG]);
+				p += N * step;
+				bp += N * KG;
+				left -= N;
+			};
+#pragma unroll 1
+			while(left >= 8) round(std::integral_constant<int, 8>{});
+			if(left >= 4) round(std::integral_constant<int, 4>{});
+			if(left >= 2) round(std::integral_constant<int, 2>{});
+			if(left >= 1) round(std::integral_constant<int, 1>{});
+		};
+		if(uniform) sum(b + k + __builtin_amdgcn_readfirstlane(kg));
+		else        sum(lb + kg);
+		__syncthreads();
+	}
+	double s[PV];
+#pragma unroll
+	for(int e = 0; e < PV; ++e) s[e] = acc[e].value();
+	if(KG > 1) {
+		for(int d = JL; d < 64; d <<= 1)
+#pragma unroll
+			for(int e = 0; e < PV; ++e) s[e] += __shfl_xor(s[e], d, 64);
+		int const w = JL < 64 ? 64 : JL;
+		int const parts = kBlock / w;
+		double* const red = reinterpret_cast<double*>(lds);
+		if((t & (w - 1)) < JL)
+#pragma unroll
+			for(int e = 0; e < PV; ++e) red[((t / w) * PV + e) * JL + jl] = s[e];
+		__syncthreads();
+		if(t >= JL) return;
+		for(int g = 1; g < parts; ++g)
+#pragma unroll
+			for(int e = 0; e < PV; ++e) s[e] += red[(g * PV + e) * JL + jl];
+	}
+	if(jl >= n) return;
+#pragma unroll
+	for(int e = 0; e < PV; ++e) store_out<double, false>(C, P, o, static_cast<int64_t>(jl) * PV + e, s[e]);
+}
+
 // (at most 96 registers: 5 waves per SIMD, as many as the LDS leaves room for)
 template<typename S, int PV, bool KAHAN>
 __global__ __launch_bounds__(kBlock, 5) void k_stage(const S* __restrict__ A, const typename Traits<S>::acc* __restrict__ b,

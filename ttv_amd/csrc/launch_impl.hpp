@@ -67,10 +67,12 @@ int launch_vec(const Config& cfg, const S* A, const typename Traits<S>::acc* B, 
 		return fail(TTVX_ERR_UNSUPPORTED, "ttvx: realigned loads for row and column products only");
 	}
 	if(cfg.lean == LEAN_LONG_ROWS) {
-		if constexpr(VEC == Traits<S>::vmax) {
+		constexpr bool F64 = std::is_same_v<S, double>;
+		if constexpr(VEC == (F64 ? 1 : Traits<S>::vmax)) {
 			dim3 const g2(static_cast<unsigned>(cfg.grid), static_cast<unsigned>(cfg.ksplit));
-			if(cfg.U == 2) hipLaunchKernelGGL((k_long_rows<S, VEC, 2, KH>), g2, block, 0, s, A, B, C, cfg.args);
-			else           hipLaunchKernelGGL((k_long_rows<S, VEC, 4, KH>), g2, block, 0, s, A, B, C, cfg.args);
+			constexpr int few = F64 ? 4 : 2, many = F64 ? 8 : 4;
+			if(cfg.U == few) hipLaunchKernelGGL((k_long_rows<S, VEC, few, KH>), g2, block, 0, s, A, B, C, cfg.args);
+			else             hipLaunchKernelGGL((k_long_rows<S, VEC, many, KH>), g2, block, 0, s, A, B, C, cfg.args);
 			return TTVX_OK;
 		}
 		return fail(TTVX_ERR_UNSUPPORTED, "ttvx: long rows take full-width vectors");

@@ -287,11 +287,13 @@ void configure_view(const Fold& f, const DType& dt, Config& cfg)
 // dot_split on three and more rows of more than one vector per lane: k_long_rows (longrows.hpp)
 bool configure_long_rows(const Fold& f, const DType& dt, Config& cfg)
 {
-	int64_t const vsteps = ceil_div(f.K, cfg.vec);
 	// one or two rows: no b to share, the looping kernel streams both operands
-	if(cfg.vec != dt.vmax || vsteps <= 64 || f.O < 3) return false;
+	if(cfg.vec != dt.vmax || ceil_div(f.K, cfg.vec) <= 64 || f.O < 3) return false;
 	Args& P = cfg.args;
-	int const n = vsteps <= 128 ? 2 : 4;
+	// FP64 by single elements, whose rows need no alignment
+	if(dt.size == 8) cfg.vec = 1;
+	int64_t const vsteps = ceil_div(f.K, cfg.vec);
+	int const n = dt.size == 8 ? (vsteps <= 256 ? 4 : 8) : (vsteps <= 128 ? 2 : 4);
 	int64_t const piece = long_piece(cfg.vec, n);
 	int64_t const pieces = ceil_div(f.K, piece);
 	// waves of a block along the row: as many as leave at most an eighth of them without a piece
@@ -461,6 +463,8 @@ bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus,
 		if(!dot_shape) return false;
 		cfg.kind = KIND_DOT;
 		cfg.vec  = pick_vec(dt, f.K);
+		// (rows: 129 elements 3.4 -> 4.7 TB/s)
+		if(v != V_DOT_SPLIT && dt.size == 8 && (a_addr % 16 != 0 || (f.O > 1 && f.sAo % 2 != 0))) cfg.vec = 1;
 		int64_t const vsteps = ceil_div(f.K, cfg.vec);
 		P.LPR = static_cast<int>(std::min<int64_t>(64, pow2_ceil(vsteps)));
 		P.lprShift = ilog2(P.LPR);
@@ -521,6 +525,12 @@ bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus,
 		int const vb = v8 ? (v == V_COL_U1_V8 ? V_COL_U1 : V_COL_U2) : v;     // the tiling it follows
 		cfg.vec  = pick_vec(dt, f.I, v8 ? 8 : 16);
 		if(v8 && (dt.size > 2 || cfg.vec == pick_vec(dt, f.I))) return false;  // nothing narrower to take
+		// FP64 tiles by single elements (8 bytes a lane, twice the lanes per row): rows off the 16-byte grid 4.5-5.1 ->
+		// 5.4-5.9 TB/s, aligned rows of 700, 2000 and 70000 3.8 -> 5.2, 4.1 -> 5.1 and 5.3 -> 5.5, of 16384 and
+		// 65536 5.9 -> 6.1 and 6.0 -> 6.2 (MI355X, contractions of 16 to 256, 0.5-2.1 GB).  col_narrow keeps pairs,
+		// whose 256-byte chunks it needs (rows of 128 6.5 against 5.2), and so does FP32: off the grid 5.2-5.9 TB/s
+		// by vectors of four, 4.9-5.6 by elements.
+		if(dt.size == 8 && vb != V_COL_NARROW) cfg.vec = 1;
 		int64_t const iv = ceil_div(f.I, cfg.vec);          // vectors per row (the last one clamped)
 		int64_t const itmax = kBlock;
 		P.IT = static_cast<int>(std::min<int64_t>(iv, itmax));

@@ -1202,6 +1202,31 @@ __device__ __forceinline__ void segment_sum(Acc (&v)[U], int kl, int len)
 	}
 }
 
+// The U row vectors of a lane at column kc of rows row0, row0 + rpw, ...  Realigned storage takes the word past its
+// vector from the next lane, which holds the row's next vector; lanes for which it does not (`edge`: the row's last
+// two vectors, the wave's last lane) load that word themselves.  @ROWX@
+template<typename S, int VEC, int U>
+__device__ __forceinline__ void row_loads(const S* __restrict__ A, const Args& P, int64_t row0, int rpw, int64_t kc,
+                                          bool edge, int lane, Vec<S, VEC> (&raw)[U])
+{
+	if constexpr(kRealigned<S> && Vec<S, VEC>::bytes >= 4) {
+		XVec<S, VEC> xr[U];
+#pragma unroll
+		for(int u = 0; u < U; ++u) {
+			int64_t const row = row0 + static_cast<int64_t>(u) * rpw;
+			xr[u].load(A + (row < P.O ? row : P.O - 1) * P.sAo + kc, edge);
+		}
+#pragma unroll
+		for(int u = 0; u < U; ++u) xr[u].finish(edge, lane, raw[u]);
+	} else {
+#pragma unroll
+		for(int u = 0; u < U; ++u) {
+			int64_t const row = row0 + static_cast<int64_t>(u) * rpw;
+			raw[u].load(A + (row < P.O ? row : P.O - 1) * P.sAo + kc);
+		}
+	}
+}
+
 // Rows of K <= 64*VEC contiguous elements (one vector per lane and row, P.kiter == 1): wave
 // blockIdx.x*4 + w sums the U*RPW rows of its group and stores their sums.  Every load is issued
 // before the first use and none sits behind a branch: lanes past the end of a row re-read the row's
@@ -1227,11 +1252,7 @@ __device__ __forceinline__ void rows_group(const S* __restrict__ A, const typena
 		load_b_vec<Acc, VEC>(b, kc, bb);
 		Vec<S, VEC> raw[U];
 		int64_t const row0 = g * U * rpw + (r < rpw ? r : 0);
-#pragma unroll
-		for(int u = 0; u < U; ++u) {
-			int64_t const row = row0 + static_cast<int64_t>(u) * rpw;
-			raw[u].load(A + (row < P.O ? row : P.O - 1) * P.sAo + kc);
-		}
+		row_loads<S, VEC, U>(A, P, row0, rpw, kc, k0 + 2 * VEC > P.K || lane == 63, lane, raw);
 		Acc v[U];
 #pragma unroll
 		for(int u = 0; u < U; ++u) {
@@ -1265,11 +1286,7 @@ __device__ __forceinline__ void rows_group(const S* __restrict__ A, const typena
 	// rows of the group: (g*U + u)*rpw + r; a group past the last row re-reads the last row
 	Vec<S, VEC> raw[U];
 	int64_t const row0 = g * U * rpw + r;
-#pragma unroll
-	for(int u = 0; u < U; ++u) {
-		int64_t const row = row0 + static_cast<int64_t>(u) * rpw;
-		raw[u].load(A + (row < P.O ? row : P.O - 1) * P.sAo + kc);
-	}
+	row_loads<S, VEC, U>(A, P, row0, rpw, kc, k0 + 2 * VEC > P.K || lane == 63, lane, raw);
 	Acc v[U];
 #pragma unroll
 	for(int u = 0; u < U; ++u) {

@@ -5,7 +5,7 @@
 // tuning table, the learned selector, the fixed rule: the same choice a single call makes) picks its
 // kernel variant, with the contraction never split.  The problem keeps that variant's configuration
 // and its block decomposition: one block per four row groups (k_rows), per 256-byte column chunk
-// item (k_slab, or run of staged slabs or rows, k_stage and k_stage_rows), per run of column items or row groups (k_col, k_dot) as the single launch's grid
+// item (k_slab, or run of staged slabs, k_stage), per run of column items or row groups (k_col, k_dot) as the single launch's grid
 // divides them.  Problems whose blocks run the same tile body (body, vector width, slab units or row
 // sets, lanes per row) form a group, and a group is ONE launch whose grid is the concatenation of
 // its problems' grids: block b reads its problem from a per-block owner table, then runs the same
@@ -34,7 +34,7 @@ namespace ttvx
 {
 
 // tile body of a group
-enum BatchBody { BB_COL = 0, BB_SLAB = 1, BB_ROWS = 2, BB_DOT = 3, BB_STAGE = 4, BB_STAGE_ROWS = 5 };
+enum BatchBody { BB_COL = 0, BB_SLAB = 1, BB_ROWS = 2, BB_DOT = 3, BB_STAGE = 4 };
 
 struct BatchDesc {
 	Args args;
@@ -89,9 +89,6 @@ __global__ __launch_bounds__(kBlock) void k_batch_group(const BatchDesc* __restr
 	} else if constexpr(BODY == BB_STAGE) {
 		extern __shared__ __attribute__((aligned(16))) unsigned char stage_lds[];
 		stage_item<float, VEC, false>(d.a, d.b, d.c, P, lb, stage_lds);
-	} else if constexpr(BODY == BB_STAGE_ROWS) {
-		extern __shared__ __attribute__((aligned(16))) unsigned char stage_lds[];
-		stage_rows_item<float, false, U == 2>(d.a, d.b, d.c, P, lb, stage_lds);
 	} else if constexpr(BODY == BB_COL) {
 		extern __shared__ unsigned char smem_raw[];
 		group_col<VEC, U>(d, P, lb, reinterpret_cast<float*>(smem_raw));
@@ -175,7 +172,6 @@ GroupKernel group_kernel(Key const& k)
 		case BB_COL:  return kernel_vec<BB_COL>(vec, U, lprc);
 		case BB_SLAB: return kernel_vec<BB_SLAB>(vec, U, lprc);
 		case BB_STAGE: return kernel_vec<BB_STAGE>(vec, U, lprc);
-		case BB_STAGE_ROWS: return U == 2 ? k_batch_group<BB_STAGE_ROWS, 1, 2, 0> : k_batch_group<BB_STAGE_ROWS, 1, 1, 0>;
 		case BB_ROWS: return kernel_vec<BB_ROWS>(vec, U, lprc);
 		default:      return kernel_vec<BB_DOT>(vec, U, lprc);
 	}
@@ -280,8 +276,8 @@ int ttvx_batch_create(size_t count, const ttvx_batch_problem* problems, void** o
 		if(cfg.lean == LEAN_SLAB) {
 			body = BB_SLAB;
 			it.blocks = cfg.args.items;
-		} else if(cfg.lean == LEAN_STAGE || cfg.lean == LEAN_STAGE_ROWS) {
-			body = cfg.lean == LEAN_STAGE ? BB_STAGE : BB_STAGE_ROWS;
+		} else if(cfg.lean == LEAN_STAGE) {
+			body = BB_STAGE;
 			it.blocks = cfg.args.items;
 		} else if(cfg.kind == KIND_COL) {
 			body = BB_COL;
@@ -302,7 +298,7 @@ int ttvx_batch_create(size_t count, const ttvx_batch_problem* problems, void** o
 		it.key = Key(body, cfg.vec, cfg.U, lprc);
 		if(group_kernel(it.key) == nullptr || cfg.shmem > 64 * 1024 || it.blocks > kMaxLeanBlocks)
 			return fail(TTVX_ERR_UNSUPPORTED, where + "tile does not fit the batched kernels");
-		it.shmem = body == BB_COL || body == BB_STAGE || body == BB_STAGE_ROWS ? cfg.shmem : 0;
+		it.shmem = body == BB_COL || body == BB_STAGE ? cfg.shmem : 0;
 		set_output_stores(cfg, f, dt, reinterpret_cast<uintptr_t>(pr.c));
 		it.d.args = cfg.args;
 		it.d.args.kchunk  = f.K;

@@ -45,8 +45,10 @@ template<typename S>
 void go_typed(const Config& cfg, const void* a, const void* b, void* c, bool kahan, hipStream_t s)
 {
 	if(cfg.lean == LEAN_STAGE_ROWS) {
-		if(cfg.args.swz) go_rows<S, true>(cfg, a, b, c, kahan, s);
-		else               go_rows<S, false>(cfg, a, b, c, kahan, s);
+		if constexpr(sizeof(S) != 4) {
+			if(cfg.args.swz) go_rows<S, true>(cfg, a, b, c, kahan, s);
+			else             go_rows<S, false>(cfg, a, b, c, kahan, s);
+		}
 	} else if(cfg.lean == LEAN_STAGE_CHUNKS) {
 		if constexpr(sizeof(S) == 8) {
 			if(cfg.vec == 2) go_chunks<2>(cfg, a, b, c, s);

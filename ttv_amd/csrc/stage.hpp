@@ -206,7 +206,7 @@ __device__ __forceinline__ void stage_item(const S* __restrict__ A, const typena
 //   513          5576 / 4390   4471 / 3213   4194 / 2955
 // Rows of whole 16-byte vectors of the 4-, 2- and 1-byte types stay with k_rows (FP8 rows of 128: 5678 / 5797), and
 // the swizzle is for rows whose starts would collide (FP8 rows of 511 without it 2.8 TB/s).
-// Rows (q fastest) in the same way: item = rows [item*OS, item*OS + OS), G = 1 << itShift neighbouring lanes per row,
+// Rows (q fastest) of FP64, BF16 and FP8 in the same way: item = rows [item*OS, item*OS + OS), G = 1 << itShift neighbouring lanes per row,
 // which take its words (of 4 bytes; 8 for FP64) in turn.  Words are read from the aligned ones that hold them, so
 // rows of 2- and 1-byte storage may start anywhere.
 template<typename S, bool KAHAN, bool SWZ>
@@ -247,9 +247,6 @@ __device__ __forceinline__ void stage_rows_item(const S* __restrict__ A, const t
 			if constexpr(sizeof(S) == 8) {
 #pragma unroll
 				for(int u = 0; u < N; ++u) x[u] = *reinterpret_cast<const double*>(lds + stage_at<SWZ>(at0 + 8 * (w + u * step)));
-			} else if constexpr(sizeof(S) == 4) {
-#pragma unroll
-				for(int u = 0; u < N; ++u) x[u] = *reinterpret_cast<const float*>(lds + stage_at<SWZ>(at0 + 4 * (w + u * step)));
 			} else {
 				uint32_t lo[N], hi[N];
 #pragma unroll

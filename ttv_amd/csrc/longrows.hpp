@@ -40,6 +40,7 @@ __global__ __launch_bounds__(kBlock) void k_long_rows(const S* __restrict__ A, c
 		// first vector and add nothing
 		int64_t kc[N];
 		int head[N];                                              // leading elements of the vector that are not this lane's
+		bool edge[N];                                             // the next lane does not hold the row's next vector
 		Acc bv[N][VEC];
 		bool const whole = k0 + long_piece(VEC, N) <= P.K;
 #pragma unroll
@@ -48,16 +49,21 @@ __global__ __launch_bounds__(kBlock) void k_long_rows(const S* __restrict__ A, c
 			bool const live = k < P.K;
 			kc[s] = live ? row_clamp(k, P.K, VEC) : 0;
 			head[s] = live ? static_cast<int>(k - kc[s]) : VEC;
+			edge[s] = lane == 63 || k + 2 * VEC > P.K;
 			load_b_vec<Acc, VEC>(b, kc[s], bv[s]);
 		}
 		// H rows at once (two in flight; an odd last one alone)
 		auto sums = [&](auto h_, int r) {
 			constexpr int H = decltype(h_)::value;
 			Vec<S, VEC> raw[H][N];
+			XVec<S, VEC> xr[H][N];            // realigned storage: the word past a vector comes from the next lane
 #pragma unroll
 			for(int h = 0; h < H; ++h)
 #pragma unroll
-				for(int s = 0; s < N; ++s) raw[h][s].load(A + (r0 + r + h) * P.sAo + kc[s]);
+				for(int s = 0; s < N; ++s) {
+					if constexpr(kRealigned<S>) xr[h][s].load(A + (r0 + r + h) * P.sAo + kc[s], edge[s]);
+					else raw[h][s].load(A + (r0 + r + h) * P.sAo + kc[s]);
+				}
 			__builtin_amdgcn_sched_barrier(0);
 			Acc v[H];
 #pragma unroll
@@ -66,6 +72,7 @@ __global__ __launch_bounds__(kBlock) void k_long_rows(const S* __restrict__ A, c
 #pragma unroll
 				for(int s = 0; s < N; ++s) {
 					Acc x[VEC];
+					if constexpr(kRealigned<S>) xr[h][s].finish(edge[s], lane, raw[h][s]);
 					decode(raw[h][s], x);
 					if(!whole)
 #pragma unroll

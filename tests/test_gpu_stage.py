@@ -112,3 +112,27 @@ def test_long_contractions(ttvx, device, I, K, Ox, dt):
             assert np.all(np.abs(C.cpu().numpy().astype(np.float64) - exact) <= (K / 8 + 64) * eps * mag + 1e-300)
     finally:
         ttvx.restore_default_selection()
+
+
+@pytest.mark.parametrize("I,K,Ox,variant", [(1, 50001, 40, SPLIT_DOT), (5, 1 << 18, 1, SPLIT_COL)])
+def test_split_under_capture_without_a_buffer(ttvx, device, I, K, Ox, variant):
+    """A capture on a stream that has no buffer for partial sums takes the unsplit kernel; every replay is right."""
+    import torch
+    A = torch.empty((Ox, K, I), device=device).uniform_(-1, 1)
+    b = torch.empty(K, device=device).uniform_(-1, 1)
+    exact = (A.double() * b.double().view(1, -1, 1)).sum(1)
+    mag = (A.double() * b.double().view(1, -1, 1)).abs().sum(1)
+    C = torch.empty((Ox, I), device=device)
+    ttvx.set_selection(ttvx.SELECT_FORCED, variant)
+    try:
+        s = torch.cuda.Stream()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            ttvx.ttv(2, A, b, out=C)
+        for _ in range(3):
+            C.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert bool(((C.double() - exact).abs() <= (K / 8 + 64) * 2.0 ** -24 * mag).all())
+    finally:
+        ttvx.restore_default_selection()

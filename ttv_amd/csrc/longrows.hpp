@@ -2,14 +2,18 @@
 //
 // A lane of the looping row kernels re-reads its values of b for every vector of A.  For 1-byte storage these are
 // 64 bytes, 64 bytes apart from lane to lane, against 16 bytes of A: the vector cache serves one lane a cycle, and
-// that, not HBM, set 2.5 TB/s (BF16: half of it, 4-5 TB/s).  Here a wave keeps the b of kLongSteps vectors per lane
-// (4 KiB of a row) and walks over the rows instead, so b is read once for `rows` of them.  WK waves of a block
-// take neighbouring pieces of the row, the other 4 / WK further rows; what a block does not cover of the
-// contraction is split over gridDim.y, with partial sums as in the split column kernel.  MI355X, 256 MiB, GB/s (before: the best looping row kernel):
-//   row length        1000          4000          20000         100003
-//   FP32              5548 -> 5837  5595 -> 5915  5418 -> 5530  4877 -> 5069
-//   BF16              5258 -> 5415  4956 -> 5985  4139 -> 5516  3433 -> 4139
-//   FP8               -             3542 -> 4676  3693 -> 4441  2507 -> 3711
+// that, not HBM, set 2.5 TB/s (BF16: half of it, 4-5 TB/s).  Here a wave keeps the b of its piece of the row (4 KiB of A
+// at most) and walks over the rows instead, so b is read once for all of them.  KS waves of a block take
+// neighbouring pieces, the other 4 / KS further rows; what a block does not cover of the contraction is split over
+// gridDim.y, with partial sums as in the split column kernel.
+//
+// MI355X, 256 MiB (rows of 4001: 240-480 MB), GB/s, before (the best looping row kernel) -> here:
+//   row length   FP32           FP64           BF16           FP8
+//   1000         5548 -> 5837   4220 -> 5311   5258 -> 5415   -
+//   4000         5595 -> 5915   3697 -> 4755   4956 -> 5985   3542 -> 4676
+//   4001         -              -              3915 -> 5698   2872 -> 3902
+//   20000        5418 -> 5530   4051 -> 4897   4139 -> 5516   3693 -> 4441
+//   100003       4877 -> 5069   3506 -> 4195   3433 -> 5575   2507 -> 3846
 // 21 rows of 4000037 FP32: 64.7 -> 58.7 us with rows in even shares (20 + 1 rows: 76 us).
 #pragma once
 

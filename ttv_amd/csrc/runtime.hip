@@ -531,7 +531,9 @@ bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus,
 		// 65536 5.9 -> 6.1 and 6.0 -> 6.2 (MI355X, contractions of 16 to 256, 0.5-2.1 GB).  col_narrow keeps pairs,
 		// whose 256-byte chunks it needs (rows of 128 6.5 against 5.2), and so does FP32: off the grid 5.2-5.9 TB/s
 		// by vectors of four, 4.9-5.6 by elements.
-		if(dt.size == 8 && vb != V_COL_NARROW) cfg.vec = 1;
+		// Split contractions over few columns keep pairs too (2, 34 and 113 columns of 256 MiB: 5.7, 4.5 and 4.1 against
+		// 5.4, 4.1 and 3.7) but for odd rows of less than two lines (3 and 7 columns: 5.0 and 4.6 against 5.3 and 4.8).
+		if(dt.size == 8 && vb != V_COL_NARROW && (vb != V_COL_SPLIT || (f.I % 2 != 0 && f.I < 32))) cfg.vec = 1;
 		int64_t const iv = ceil_div(f.I, cfg.vec);          // vectors per row (the last one clamped)
 		int64_t const itmax = kBlock;
 		P.IT = static_cast<int>(std::min<int64_t>(iv, itmax));
@@ -633,6 +635,12 @@ bool configure(int v, const Fold& f, const DType& dt, uintptr_t a_addr, int cus,
 		else P.red = 2;
 		cfg.shmem = P.red == 2 ? static_cast<std::size_t>(cfg.U) * cfg.vec * kBlock * acc_size(dt) : 0;
 		if(cfg.shmem > 64 * 1024) return false;
+		// FP32 chains of more than 512 sums per lane: cut where 32 KiB of LDS hold the block's sums
+		std::size_t const sums = static_cast<std::size_t>(cfg.U) * cfg.vec * kBlock * sizeof(float);
+		if(dt.size < 8 && std::min(P.K, P.kchunk) / P.KS > 512 && sums <= 32 * 1024) {
+			P.flush = 16;
+			cfg.shmem = std::max(cfg.shmem, sums);
+		}
 		P.one_step = (P.red != 2 && P.kchunk <= P.KS && P.K <= P.KS) ? 1 : 0;
 	}
 	if(fp64_final && dt.code != TTVX_F64) P.part64 = 1;
@@ -858,13 +866,15 @@ int launch(const Fold& f, const DType& dt, const void* a, const void* b, void* c
 		if(!configure(variant, f, dt, a_addr, di.cus, flags, cfg))
 			return fail(TTVX_ERR_UNSUPPORTED, "ttvx: no kernel variant can run this problem");
 	}
-	// products that one pass can do as well do not split where their partial sums exceed the caller's scratch or
-	// would need an allocation that a capture forbids
-	if((cfg.lean == LEAN_LONG_ROWS || cfg.lean == LEAN_STAGE_CHUNKS) && cfg.ksplit > 1) {
+	// a contraction is not split where its partial sums would need an allocation that a capture forbids, nor, by the
+	// kernels that split more than they have to, where they exceed the caller's scratch
+	if(cfg.ksplit > 1) {
 		std::size_t const bytes = static_cast<std::size_t>(cfg.ksplit) * static_cast<std::size_t>(f.O * f.I) *
 		                          (cfg.args.part64 ? 8 : acc_size(dt));
-		if(scratch != nullptr ? bytes > scratch->bytes : !partial_buffer_ready(di.id, stream, bytes) && capturing(stream))
-			configure(cfg.lean == LEAN_LONG_ROWS ? V_DOT_U2 : V_COL_U1, f, dt, a_addr, di.cus, flags, cfg);
+		bool const unsplit = scratch != nullptr
+		                         ? (cfg.lean == LEAN_LONG_ROWS || cfg.lean == LEAN_STAGE_CHUNKS) && bytes > scratch->bytes
+		                         : !partial_buffer_ready(di.id, stream, bytes) && capturing(stream);
+		if(unsplit) configure(cfg.kind == KIND_DOT ? V_DOT_U2 : V_COL_U1, f, dt, a_addr, di.cus, flags, cfg);
 	}
 	bool const kahan = (flags & TTVX_FLAG_KAHAN) != 0;
 	set_output_stores(cfg, f, dt, reinterpret_cast<uintptr_t>(c));

@@ -61,10 +61,9 @@ struct DType {
 };
 DType dtype_of(int code);
 
-// Kernels of the one-wave-per-group regime (kernels.hpp): k_rows for rows of one vector per lane,
-// k_slab for col_narrow (k_stage, stage.hpp, where slabs are small), k_stage_rows for col_k_lanes on short rows,
-// k_long_rows (longrows.hpp) for dot_split, k_stage_chunks for col_split on rows of up to a few KiB; LEAN_NONE for the looping k_dot / k_col / k_strided.  Views that do not fold:
-// k_view_cols / k_view_rows / k_view_long_rows (view.hpp).
+// Kernels behind a variant besides the looping k_dot / k_col / k_strided (LEAN_NONE): k_rows for rows of one vector per
+// lane (LEAN_ROWS), k_slab for col_narrow (LEAN_SLAB); views that do not fold (view.hpp); LDS-staged slabs for
+// col_narrow, rows for col_k_lanes and FP64 chunks for col_split (stage.hpp); long rows for dot_split (longrows.hpp).
 enum Lean {
 	LEAN_NONE = 0, LEAN_ROWS = 1, LEAN_SLAB = 2,
 	LEAN_VIEW_COLS = 3, LEAN_VIEW_ROWS = 4, LEAN_VIEW_LONG_ROWS = 5,

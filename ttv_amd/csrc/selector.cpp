@@ -31,8 +31,8 @@ using TKey = std::tuple<int, int64_t, int64_t, int64_t>;
 std::map<TKey, int> g_table;
 bool g_table_decided = false;
 // decision cache of folded 3-D problems: (dtype, O, K, I, alignment class, qpos, p, stride class)
-// -> variant; the stride class (unit k stride, unit i strides of A and C) is what decides which
-// variants can run a folded problem besides its extents
+// -> variant; the stride class (unit k stride, unit i strides of A and C, no gaps) is what decides which
+// variants can run a folded problem, and by which kernel, besides its extents
 using Key = std::tuple<int, int64_t, int64_t, int64_t, int, int, int, int>;
 std::map<Key, int> g_cache;
 } // namespace
@@ -192,13 +192,29 @@ int set_selector_table(const int64_t* rows, std::size_t count)
 	return TTVX_OK;
 }
 
+namespace
+{
+// The timings behind the table and the network are of tensors without gaps.  Whether variant v, which on such a tensor
+// of these extents runs an LDS-staged kernel, runs another one on this problem's strides: then its timing says nothing.
+bool staged_elsewhere(int v, const Fold& f, const DType& dt, uintptr_t a_addr, unsigned flags, const Config& here)
+{
+	if(v != V_COL_NARROW && v != V_COL_K_LANES && v != V_COL_SPLIT) return false;
+	Fold dense = f;
+	dense.sAk = f.I > 1 ? f.I : 1;
+	dense.sAo = f.K * f.I;
+	Config cfg;
+	return configure(v, dense, dt, a_addr, 256, flags, cfg) && cfg.lean != here.lean;
+}
+} // namespace
+
 int learned_variant(const Fold& f, const DType& dt, uintptr_t a_addr, unsigned flags)
 {
 	// problems that do not fold run the strided kernel whatever the network says
 	if(!f.three_d) return -1;
 	std::shared_ptr<const std::vector<float>> w;
 	int const align = static_cast<int>(a_addr % 16);
-	int const strides = (f.sAk == 1 ? 1 : 0) | (f.sAi == 1 ? 2 : 0) | (f.sCi == 1 ? 4 : 0);
+	int const strides = (f.sAk == 1 ? 1 : 0) | (f.sAi == 1 ? 2 : 0) | (f.sCi == 1 ? 4 : 0) |
+	                    (f.sAk == f.I && (f.O == 1 || f.sAo == f.K * f.I) ? 8 : 0);
 	Key const key{dt.code, f.O, f.K, f.I, align, f.qpos, f.p, strides};
 	{
 		std::lock_guard<std::mutex> lock(g_sel_mutex);
@@ -208,7 +224,8 @@ int learned_variant(const Fold& f, const DType& dt, uintptr_t a_addr, unsigned f
 		if(f.three_d && align == 0) {
 			auto t = g_table.find(TKey{dt.code, f.O, f.K, f.I});
 			Config cfg;
-			if(t != g_table.end() && configure(t->second, f, dt, a_addr, 256, flags, cfg)) {
+			if(t != g_table.end() && configure(t->second, f, dt, a_addr, 256, flags, cfg) &&
+			   !staged_elsewhere(t->second, f, dt, a_addr, flags, cfg)) {
 				if(g_cache.size() > 4096) g_cache.clear();
 				g_cache[key] = t->second;
 				return t->second;
@@ -227,6 +244,7 @@ int learned_variant(const Fold& f, const DType& dt, uintptr_t a_addr, unsigned f
 	Config cfg;
 	for(int v = 0; v < kMlpV; ++v) {
 		if(v == V_STRIDED || !configure(v, f, dt, a_addr, 256, flags, cfg)) continue;
+		if(staged_elsewhere(v, f, dt, a_addr, flags, cfg)) continue;
 		if(best < 0 || y[v] < y[best]) best = v;
 	}
 	if(best < 0 && configure(V_STRIDED, f, dt, a_addr, 256, flags, cfg)) best = V_STRIDED;

@@ -227,11 +227,17 @@ def shapes_from_arrays(z):
 
 # ---- training on the GPU --------------------------------------------------------------------
 
+# Predicted slowdowns end at 2^0.5: how much slower than that a variant is decides nothing, and without the bound those
+# errors were most of the loss (held-out regret 1.9 % -> 1.5 % with it and 1000 instead of 300 epochs).
+MOST_SLOWDOWN = 0.5
+
+
 def targets(times):
-    """log2 slowdown vs the fastest variant, and the validity mask."""
+    """log2 slowdown vs the fastest variant (at most MOST_SLOWDOWN), and the validity mask."""
     best = np.nanmin(times, axis=1, keepdims=True)
     mask = np.isfinite(times).astype(np.float32)
-    t = np.where(mask > 0, np.log2(np.where(mask > 0, times, 1.0) / best), 0.0).astype(np.float32)
+    t = np.where(mask > 0, np.log2(np.where(mask > 0, times, 1.0) / best), 0.0)
+    t = np.minimum(t, MOST_SLOWDOWN).astype(np.float32)
     return t, mask
 
 
@@ -281,7 +287,7 @@ class GPUTrainer:
                                   0.999, 1e-8, wd, _stream()))
 
 
-def train(feats, times, epochs=300, batch=512, lr=2e-3, seed=0, log=None, n_structured=0, struct_weight=1):
+def train(feats, times, epochs=1000, batch=512, lr=2e-3, seed=0, log=None, n_structured=0, struct_weight=1):
     """Adam on the GPU kernels; the last n_structured rows (benchmark shapes) are repeated
     struct_weight times, so the common benchmark shapes weigh more than one random shape each."""
     import torch
@@ -304,7 +310,7 @@ def train(feats, times, epochs=300, batch=512, lr=2e-3, seed=0, log=None, n_stru
         for k in range(nb):
             idx = perm[k * batch:(k + 1) * batch]
             tr.step(X[idx].contiguous(), Td[idx].contiguous(), Md[idx].contiguous(), float(lr_ep))
-        if log and (ep + 1) % 50 == 0:
+        if log and (ep + 1) % 100 == 0:
             torch.cuda.synchronize()
             log("epoch %d loss %.4f" % (ep + 1, float(tr.loss.item())))
     torch.cuda.synchronize()
@@ -381,7 +387,7 @@ def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--train", type=int, default=20000)
     ap.add_argument("--test", type=int, default=2000)
-    ap.add_argument("--epochs", type=int, default=300)
+    ap.add_argument("--epochs", type=int, default=1000)
     ap.add_argument("--reps", type=int, default=3)
     ap.add_argument("--out", default="selector_out")
     ap.add_argument("--tables", help="directory with timings_train.npz / timings_test.npz to train on")

@@ -232,6 +232,33 @@ def test_batch_graph_replays(ttvx, device):
     bt.close()
 
 
+@pytest.mark.parametrize("cap", [1 << 12, 1 << 18, 1 << 22])
+def test_batch_small_groups_join(ttvx, device, cap):
+    """A batch that picks its variants itself takes at most a few launches when its groups are small: no more than
+    the same problems with each one's single-call variant named; single outputs bit for bit, and the oracle."""
+    import torch
+    from ttv_amd.batch import Batch
+    rng = np.random.default_rng(cap)
+    specs = []
+    while len(specs) < 16:
+        p = int(rng.integers(2, 5))
+        na = [int(rng.integers(2, 200)) for _ in range(p)]
+        if np.prod(na) <= cap:
+            specs.append(_spec(na, int(rng.integers(1, p + 1)), [int(m) + 1 for m in rng.permutation(p)]))
+    probs = _make(torch, device, specs, 21)
+    own = [ttvx.plan_info(q, s["na"], s["wa"], s["pia"])["variant"] for (q, _, _), s in zip(probs, specs)]
+    bt, named = Batch(probs), Batch(probs, variants=own)
+    assert bt.info()["launches"] <= named.info()["launches"]
+    bt.launch(graph=False)
+    torch.cuda.synchronize()
+    batched = [_flat(C).cpu().numpy().copy() for C in bt.outputs]
+    _check_against_single(ttvx, bt, probs, batched)
+    for n, (q, A, b) in enumerate(probs):
+        _check_oracle(q, A, b, bt.outputs[n], batched[n])
+    named.close()
+    bt.close()
+
+
 def test_batch_rejects_bad_problems(ttvx, device):
     import torch
     from ttv_amd.batch import Batch

@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <map>
 #include <tuple>
@@ -100,6 +101,10 @@ __global__ __launch_bounds__(kBlock) void k_batch_group(const BatchDesc* __restr
 namespace
 {
 using GroupKernel = void (*)(const BatchDesc*, const uint32_t*);
+
+constexpr double kGroupCost  = 4e-6;      // s; a further launch of a batch, measured between batches of 5 to 9 launches
+constexpr double kStreamRate = 5e12;      // byte/s of a mid-size launch
+constexpr float kKnownSlowdown = 0.4f;    // log2
 
 // group key: body, vector width, slab units / row sets, lanes per row fixed at compile time
 using Key = std::tuple<int, int, int, int>;
@@ -239,39 +244,14 @@ int ttvx_batch_create(size_t count, const ttvx_batch_problem* problems, void** o
 		std::size_t shmem;
 		int64_t cost;
 	};
-	std::vector<Item> items;
-	items.reserve(count);
-	std::vector<int> variant(count, -1);
-	int64_t bytes = 0;
-	for(size_t n = 0; n < count; ++n) {
-		ttvx_batch_problem const& pr = problems[n];
-		std::string const where = "ttvx_batch_create: problem " + std::to_string(n) + ": ";
-		Check ck = validate_a(pr.q, pr.p, pr.na, pr.wa, pr.pia);
-		if(ck.status != TTVX_OK) return fail(ck.status, where + ck.message);
-		if(pr.p < 2) return fail(TTVX_ERR_ARGUMENT, where + "Error in tlib::tensor_times_vector: shape vector of C is not valid.");
-		if(pr.a == nullptr || pr.b == nullptr || pr.c == nullptr) return fail(TTVX_ERR_ARGUMENT, where + "null data pointer");
-		Fold const f = fold(pr.q, pr.p, pr.na, pr.wa, pr.pia, pr.wc, nullptr);
-		int rc = check_device_span(pr.a, static_cast<size_t>(f.a_span) * 4, "A");
-		if(rc == TTVX_OK) rc = check_device_span(pr.b, static_cast<size_t>(f.K) * 4, "b");
-		if(rc == TTVX_OK) rc = check_device_span(pr.c, static_cast<size_t>(f.c_span) * 4, "C");
-		if(rc != TTVX_OK) return fail(rc, where + ttvx_last_error());
-		if(f.K > (int64_t{1} << 20))
-			return fail(TTVX_ERR_UNSUPPORTED, where + "the batched kernel does not split contractions longer than 2^20; "
-			                                          "run such products alone (they use an FP64 final reduction)");
+	// the tile of problem pr under variant v, unsplit; TILE_UNFIT where no group kernel holds it
+	enum { TILE_OK, TILE_INVALID, TILE_UNFIT };
+	auto tile = [&](ttvx_batch_problem const& pr, Fold const& f, int v, Item& it) -> int {
 		uintptr_t const aaddr = reinterpret_cast<uintptr_t>(pr.a);
-		// the problem's own variant, or the one a single call would take; the contraction is never split
-		if(pr.variant >= ttvx_num_variants())
-			return fail(TTVX_ERR_ARGUMENT, where + "no kernel variant " + std::to_string(pr.variant));
-		int v = pr.variant >= 0 ? pr.variant : select_variant(f, dt, aaddr, 0u);
-		if(v == V_COL_SPLIT) v = V_COL_U1;
-		if(v == V_DOT_SPLIT) v = V_DOT_U2;
 		Config cfg;
 		if(v == V_STRIDED || !configure(v, f, dt, aaddr, di.cus, 0u, cfg) || cfg.ksplit != 1 || cfg.args.part64)
-			return fail(TTVX_ERR_UNSUPPORTED, where + (pr.variant >= 0 ? std::string("variant ") + ttvx_variant_name(pr.variant) +
-			                                                            " cannot run this problem in a batch"
-			                                                          : std::string("the batched kernel needs A and C to fold "
-			                                                                        "to three dense-inner dimensions")));
-		Item it{};
+			return TILE_INVALID;
+		it = Item{};
 		int body, lprc = 0;
 		if(cfg.lean == LEAN_SLAB) {
 			body = BB_SLAB;
@@ -297,7 +277,7 @@ int ttvx_batch_create(size_t count, const ttvx_batch_problem* problems, void** o
 		}
 		it.key = Key(body, cfg.vec, cfg.U, lprc);
 		if(group_kernel(it.key) == nullptr || cfg.shmem > 64 * 1024 || it.blocks > kMaxLeanBlocks)
-			return fail(TTVX_ERR_UNSUPPORTED, where + "tile does not fit the batched kernels");
+			return TILE_UNFIT;
 		it.shmem = body == BB_COL || body == BB_STAGE ? cfg.shmem : 0;
 		set_output_stores(cfg, f, dt, reinterpret_cast<uintptr_t>(pr.c));
 		it.d.args = cfg.args;
@@ -311,6 +291,53 @@ int ttvx_batch_create(size_t count, const ttvx_batch_problem* problems, void** o
 		it.d.b = pr.b;
 		it.d.c = pr.c;
 		it.cost = f.outputs * f.K;
+		return TILE_OK;
+	};
+	auto unsplit = [](int v) { return v != V_COL_SPLIT && v != V_DOT_SPLIT; };
+	std::vector<Item> items;
+	items.reserve(count);
+	std::vector<int> variant(count, -1);
+	int64_t bytes = 0;
+	for(size_t n = 0; n < count; ++n) {
+		ttvx_batch_problem const& pr = problems[n];
+		std::string const where = "ttvx_batch_create: problem " + std::to_string(n) + ": ";
+		Check ck = validate_a(pr.q, pr.p, pr.na, pr.wa, pr.pia);
+		if(ck.status != TTVX_OK) return fail(ck.status, where + ck.message);
+		if(pr.p < 2) return fail(TTVX_ERR_ARGUMENT, where + "Error in tlib::tensor_times_vector: shape vector of C is not valid.");
+		if(pr.a == nullptr || pr.b == nullptr || pr.c == nullptr) return fail(TTVX_ERR_ARGUMENT, where + "null data pointer");
+		Fold const f = fold(pr.q, pr.p, pr.na, pr.wa, pr.pia, pr.wc, nullptr);
+		int rc = check_device_span(pr.a, static_cast<size_t>(f.a_span) * 4, "A");
+		if(rc == TTVX_OK) rc = check_device_span(pr.b, static_cast<size_t>(f.K) * 4, "b");
+		if(rc == TTVX_OK) rc = check_device_span(pr.c, static_cast<size_t>(f.c_span) * 4, "C");
+		if(rc != TTVX_OK) return fail(rc, where + ttvx_last_error());
+		if(f.K > (int64_t{1} << 20))
+			return fail(TTVX_ERR_UNSUPPORTED, where + "the batched kernel does not split contractions longer than 2^20; "
+			                                          "run such products alone (they use an FP64 final reduction)");
+		uintptr_t const aaddr = reinterpret_cast<uintptr_t>(pr.a);
+		// the problem's own variant, or the one a single call would take; the contraction is never split
+		if(pr.variant >= ttvx_num_variants())
+			return fail(TTVX_ERR_ARGUMENT, where + "no kernel variant " + std::to_string(pr.variant));
+		int v = pr.variant >= 0 ? pr.variant : select_variant(f, dt, aaddr, 0u);
+		// a pick that splits gives way to the one predicted fastest of the others
+		float slow[V_COUNT];
+		if(!unsplit(v) && pr.variant < 0 && learned_selection() &&
+		   predicted_slowdowns(f, dt, aaddr, 0u, slow)) {
+			Item it;
+			int u = -1;
+			for(int w = 0; w < V_COUNT; ++w)
+				if(unsplit(w) && slow[w] < kKnownSlowdown && (u < 0 || slow[w] < slow[u]) && tile(pr, f, w, it) == TILE_OK) u = w;
+			if(u >= 0) v = u;
+		}
+		if(v == V_COL_SPLIT) v = V_COL_U1;
+		if(v == V_DOT_SPLIT) v = V_DOT_U2;
+		Item it;
+		int const t = tile(pr, f, v, it);
+		if(t == TILE_INVALID)
+			return fail(TTVX_ERR_UNSUPPORTED, where + (pr.variant >= 0 ? std::string("variant ") + ttvx_variant_name(pr.variant) +
+			                                                            " cannot run this problem in a batch"
+			                                                          : std::string("the batched kernel needs A and C to fold "
+			                                                                        "to three dense-inner dimensions")));
+		if(t == TILE_UNFIT) return fail(TTVX_ERR_UNSUPPORTED, where + "tile does not fit the batched kernels");
 		variant[n] = v;
 		items.push_back(it);
 		bytes += f.outputs * f.K * 4 + f.outputs * 4 + f.K * 4;
@@ -321,6 +348,54 @@ int ttvx_batch_create(size_t count, const ttvx_batch_problem* problems, void** o
 	// continues in another launch
 	std::map<Key, std::vector<int>> groups;
 	for(size_t n = 0; n < items.size(); ++n) groups[items[n].key].push_back(static_cast<int>(n));
+
+	// A group is a launch, and a launch of its own takes kGroupCost: a group whose problems, each by the fastest
+	// variant of a group that is there anyway, lose less time than that joins those groups, the smallest group
+	// first.  A problem's loss is its predicted slowdown times its bytes' time.  Predictions near the 2^0.5 at which
+	// the network's slowdowns end are not taken for one.  Variants named by the caller stay.  Measured, every problem
+	// in its own variant's group against joined groups: 9 products of 185 MB 56.3 -> 49.2 us, 23 of 440 MB 117.6 ->
+	// 102.6, 28 of 124 MB 66.0 -> 61.8, 48 of 4.6 GB 852 -> 843.
+	if(learned_selection()) {
+		std::vector<std::pair<int64_t, Key>> order;
+		for(auto const& g : groups) {
+			int64_t cost = 0;
+			for(int m : g.second) cost += items[m].cost;
+			order.emplace_back(cost, g.first);
+		}
+		std::sort(order.begin(), order.end());
+		for(auto const& o : order) {
+			if(groups.size() == 1) break;
+			std::vector<int> const members = groups[o.second];
+			std::vector<std::pair<Item, int>> moved;
+			double loss = 0;
+			for(int m : members) {
+				ttvx_batch_problem const& pr = problems[m];
+				Fold const f = fold(pr.q, pr.p, pr.na, pr.wa, pr.pia, pr.wc, nullptr);
+				float slow[V_COUNT];
+				if(pr.variant >= 0 || !predicted_slowdowns(f, dt, reinterpret_cast<uintptr_t>(pr.a), 0u, slow)) break;
+				Item best{};
+				int bv = -1;
+				for(int v = 0; v < V_COUNT; ++v) {
+					Item it;
+					if(!unsplit(v) || slow[v] >= kKnownSlowdown || (bv >= 0 && slow[v] >= slow[bv])) continue;
+					if(tile(pr, f, v, it) != TILE_OK || it.key == o.second || groups.count(it.key) == 0) continue;
+					best = it;
+					bv = v;
+				}
+				if(bv < 0) break;
+				loss += std::max(0.f, std::exp2(slow[bv]) - 1.f) * 4.0 * static_cast<double>(items[m].cost) / kStreamRate;
+				if(loss >= kGroupCost) break;
+				moved.emplace_back(best, bv);
+			}
+			if(moved.size() != members.size()) continue;
+			groups.erase(o.second);
+			for(size_t j = 0; j < members.size(); ++j) {
+				items[members[j]] = moved[j].first;
+				variant[members[j]] = moved[j].second;
+				groups[moved[j].first.key].push_back(members[j]);
+			}
+		}
+	}
 	struct Plan {
 		Key key;
 		std::vector<int> members;

@@ -701,6 +701,12 @@ int set_selection(int mode, int forced)
 	return TTVX_OK;
 }
 
+bool learned_selection()
+{
+	int const mode = g_sel_mode.load();
+	return mode == TTVX_SELECT_LEARNED || mode == TTVX_SELECT_AUTO;
+}
+
 int select_variant(const Fold& f, const DType& dt, uintptr_t a_addr, unsigned flags)
 {
 	int const mode = g_sel_mode.load();

@@ -108,6 +108,12 @@ void features_of(const Fold& f, const DType& dt, uintptr_t a_addr, float* out);
 // when no weights are loaded.
 int learned_variant(const Fold& f, const DType& dt, uintptr_t a_addr, unsigned flags);
 
+// The MLP's log2 slowdown of every variant against the fastest (V_COUNT floats), infinite for those that cannot run
+// the problem; false when no weights are loaded.
+bool predicted_slowdowns(const Fold& f, const DType& dt, uintptr_t a_addr, unsigned flags, float* y);
+// Whether the process-wide selection mode asks the network.
+bool learned_selection();
+
 // Loads/clears the learned selector's weights (layout in mlp.hpp); count 0 clears.
 int set_selector_weights(const float* params, std::size_t count);
 // Loads the shipped selector weights once per process unless weights were set (or cleared)

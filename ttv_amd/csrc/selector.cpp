@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <limits>
 #include <string>
 #include <map>
 #include <memory>
@@ -205,6 +206,19 @@ bool staged_elsewhere(int v, const Fold& f, const DType& dt, uintptr_t a_addr, u
 	Config cfg;
 	return configure(v, dense, dt, a_addr, 256, flags, cfg) && cfg.lean != here.lean;
 }
+
+// The network's log2 slowdown of each variant against the fastest; infinite where a variant cannot run the problem or
+// its timing says nothing of it.
+void predict(const std::vector<float>& w, const Fold& f, const DType& dt, uintptr_t a_addr, unsigned flags, float* y)
+{
+	float x[kMlpF];
+	features_of(f, dt, a_addr, x);
+	mlp_forward_host(w.data(), x, y);
+	Config cfg;
+	for(int v = 0; v < kMlpV; ++v)
+		if(v == V_STRIDED || !configure(v, f, dt, a_addr, 256, flags, cfg) || staged_elsewhere(v, f, dt, a_addr, flags, cfg))
+			y[v] = std::numeric_limits<float>::infinity();
+}
 } // namespace
 
 int learned_variant(const Fold& f, const DType& dt, uintptr_t a_addr, unsigned flags)
@@ -234,24 +248,32 @@ int learned_variant(const Fold& f, const DType& dt, uintptr_t a_addr, unsigned f
 		w = g_weights;
 		if(!w) return -1;
 	}
-	float x[kMlpF], y[kMlpV];
-	features_of(f, dt, a_addr, x);
-	mlp_forward_host(w->data(), x, y);
 	// argmin of the predicted slowdown over the variants that can run the shape; the strided
 	// fallback is never timed for the training set when a dense variant exists, so it is only
 	// taken when nothing else can run
+	float y[kMlpV];
+	predict(*w, f, dt, a_addr, flags, y);
 	int best = -1;
+	for(int v = 0; v < kMlpV; ++v)
+		if(std::isfinite(y[v]) && (best < 0 || y[v] < y[best])) best = v;
 	Config cfg;
-	for(int v = 0; v < kMlpV; ++v) {
-		if(v == V_STRIDED || !configure(v, f, dt, a_addr, 256, flags, cfg)) continue;
-		if(staged_elsewhere(v, f, dt, a_addr, flags, cfg)) continue;
-		if(best < 0 || y[v] < y[best]) best = v;
-	}
 	if(best < 0 && configure(V_STRIDED, f, dt, a_addr, 256, flags, cfg)) best = V_STRIDED;
 	std::lock_guard<std::mutex> lock(g_sel_mutex);
 	if(g_cache.size() > 4096) g_cache.clear();
 	g_cache[key] = best;
 	return best;
+}
+
+bool predicted_slowdowns(const Fold& f, const DType& dt, uintptr_t a_addr, unsigned flags, float* y)
+{
+	std::shared_ptr<const std::vector<float>> w;
+	{
+		std::lock_guard<std::mutex> lock(g_sel_mutex);
+		w = g_weights;
+	}
+	if(!w || !f.three_d) return false;
+	predict(*w, f, dt, a_addr, flags, y);
+	return true;
 }
 
 } // namespace ttvx
